@@ -669,15 +669,13 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2)
             *(float4 *)(attn + rowoff + 32 * dt + 8 * r4 + 4 * hh) =
                 make_float4(y[4 * r4], y[4 * r4 + 1], y[4 * r4 + 2], y[4 * r4 + 3]);
         if (qs) {
-            int qv[16];
+            uint32_t qv[4];
             uint16_t dbits;
             int sum;
             quant_block_pair16(y, qv, dbits, sum);
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4)
-                *(uint32_t *)(qs + rowoff + 32 * dt + 8 * r4 + 4 * hh) =
-                    (uint32_t)(qv[4 * r4] & 0xff) | (uint32_t)(qv[4 * r4 + 1] & 0xff) << 8 |
-                    (uint32_t)(qv[4 * r4 + 2] & 0xff) << 16 | (uint32_t)(qv[4 * r4 + 3] & 0xff) << 24;
+                *(uint32_t *)(qs + rowoff + 32 * dt + 8 * r4 + 4 * hh) = qv[r4];
             if (hh == 0) {
                 const size_t bi = (rowoff + 32 * dt) / SI_QK;
                 qd[bi] = dbits;

@@ -43,35 +43,6 @@ struct Q8Lds {
     int16_t *s;
 };
 
-// quantize_q8 of one block held by one thread (bit-exact, same rules as
-// quant_block_lane).
-__device__ __forceinline__ void quant_block_serial(const float (&v)[32], uint32_t (&q)[8],
-                                                   uint16_t &dbits, int &bsum) {
-    float amax = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) amax = fmaxf(amax, fabsf(v[j]));  // NaN ignored
-    const float d = __fdiv_rn(amax, 127.0f);
-    dbits = f2h(d);
-    const float inv = (d == 0.0f) ? 0.0f : __fdiv_rn(1.0f, d);
-    int sum = 0;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) q[j] = 0;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) {
-        const float y = __fmul_rn(v[j], inv);
-        int qq;
-        if (!(fabsf(y) <= 3.0e38f)) {
-            qq = -127;  // NaN or +-inf: lrintf gives LONG_MIN on x86-64
-        } else {
-            qq = (int)rintf(fminf(fmaxf(y, -200.0f), 200.0f));
-            qq = qq > 127 ? 127 : (qq < -127 ? -127 : qq);
-        }
-        sum += qq;
-        q[j >> 2] |= (uint32_t)(qq & 0xff) << (8 * (j & 3));
-    }
-    bsum = sum;
-}
-
 // RMSNorm (qwen_one_layer.c:164-169) then quantize_q8 (:98-116) of one
 // activation row into LDS.  Thread t owns 4 consecutive values (t + T*i
 // groups of 4), so a Q8 block is 8 consecutive lanes and its max and sum
@@ -365,7 +336,7 @@ __global__ void __launch_bounds__(T) k_dec_gateup(
     if (t & 32) return;  // lanes 0..31 of each wavefront hold the gate rows
     // SwiGLU (silu(g) = g / (1 + e^-g), then * u) and quantize_q8 of the block
     const float gv = y, u = L.y[t + 32];
-    const float a = __fmul_rn(__fdiv_rn(gv, __fadd_rn(1.0f, expf(-gv))), u);
+    const float a = swiglu(gv, u);
     uint16_t dbits;
     int bsum;
     const int q = quant_block_lane(a, dbits, bsum);

@@ -377,8 +377,7 @@ __device__ __forceinline__ void gemm_tile_epilogue(
             for (int v = 0; v < 16; ++v) {
                 const int i = 8 * (v >> 2) + 4 * g + (v & 3);
                 const float gv = acc[a][0][v] * os, uv = acc[a][TN - 1][v] * os;
-                const float silu = __fdiv_rn(gv, __fadd_rn(1.0f, expf(-gv)));
-                tl[i * FT + j] = __fmul_rn(silu, uv);
+                tl[i * FT + j] = swiglu(gv, uv);
                 if (out && r0 + i < m && fok) {
                     out[(size_t)(r0 + i) * ldo + fb + j] = gv;
                     out[(size_t)(r0 + i) * ldo + f + fb + j] = uv;
@@ -396,10 +395,10 @@ __device__ __forceinline__ void gemm_tile_epilogue(
                 x[4 * t + 3] = p.w;
             }
             __builtin_amdgcn_wave_barrier();  // the next tile rewrites the area
-            int q[16];
+            uint32_t pk[4];
             uint16_t dbits;
             int bsum;
-            quant_block_pair16(x, q, dbits, bsum);
+            quant_block_pair16(x, pk, dbits, bsum);
             const int row = r0 + rr;
             if (row < m && fok) {
                 const size_t o = (size_t)row * f + fb + 16 * hh;
@@ -408,11 +407,6 @@ __device__ __forceinline__ void gemm_tile_epilogue(
                     for (int t = 0; t < 4; ++t)
                         *(float4 *)(go.act + o + 4 * t) =
                             make_float4(x[4 * t], x[4 * t + 1], x[4 * t + 2], x[4 * t + 3]);
-                uint32_t pk[4];
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    pk[t] = (uint32_t)(q[4 * t] & 0xff) | (uint32_t)(q[4 * t + 1] & 0xff) << 8 |
-                            (uint32_t)(q[4 * t + 2] & 0xff) << 16 | (uint32_t)q[4 * t + 3] << 24;
                 *(uint4 *)(go.qs + o) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
                 if (hh == 0) {
                     go.d[o / SI_QK] = dbits;
@@ -1089,8 +1083,7 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm_h16(
             for (int v = 0; v < 16; ++v) {
                 const int i = 8 * (v >> 2) + 4 * g + (v & 3);
                 const float gv = acc[a][0][v], uv = acc[a][TN - 1][v];
-                const float silu = __fdiv_rn(gv, __fadd_rn(1.0f, expf(-gv)));
-                tl[i * FT + j] = __fmul_rn(silu, uv);
+                tl[i * FT + j] = swiglu(gv, uv);
                 if (out && r0 + i < m && fok) {
                     out[(size_t)(r0 + i) * ldo + fb + j] = gv;
                     out[(size_t)(r0 + i) * ldo + f + fb + j] = uv;
@@ -1107,10 +1100,10 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm_h16(
                 x[4 * t + 3] = p.w;
             }
             __builtin_amdgcn_wave_barrier();
-            int q[16];
+            uint32_t pk[4];
             uint16_t dbits;
             int bsum;
-            quant_block_pair16(x, q, dbits, bsum);
+            quant_block_pair16(x, pk, dbits, bsum);
             const int row = r0 + rr;
             if (row < m && fok) {
                 const size_t o = (size_t)row * f + fb + 16 * hh;
@@ -1119,11 +1112,6 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm_h16(
                     for (int t = 0; t < 4; ++t)
                         *(float4 *)(go.act + o + 4 * t) =
                             make_float4(x[4 * t], x[4 * t + 1], x[4 * t + 2], x[4 * t + 3]);
-                uint32_t pk[4];
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    pk[t] = (uint32_t)(q[4 * t] & 0xff) | (uint32_t)(q[4 * t + 1] & 0xff) << 8 |
-                            (uint32_t)(q[4 * t + 2] & 0xff) << 16 | (uint32_t)q[4 * t + 3] << 24;
                 *(uint4 *)(go.qs + o) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
                 if (hh == 0) {
                     go.d[o / SI_QK] = dbits;
@@ -1595,8 +1583,7 @@ __global__ void __launch_bounds__(64 * BD_W) k_gemm_bd(
     // features of the row's block)
     auto gateup_out = [&](int row, int feat, float gv, float uv) {
         const int f = go.f;
-        const float silu = __fdiv_rn(gv, __fadd_rn(1.0f, expf(-gv)));
-        const float av = __fmul_rn(silu, uv);
+        const float av = swiglu(gv, uv);
         uint16_t dbits;
         int bsum;
         const int qv = quant_block_lane(av, dbits, bsum);  // all 32 lanes of the half
@@ -1798,8 +1785,7 @@ __global__ void __launch_bounds__(256) k_gemm_reduce_swiglu_q8(
         gu[og] = g;
         gu[ou] = u;
     }
-    const float silu = __fdiv_rn(g, __fadd_rn(1.0f, expf(-g)));
-    const float a = __fmul_rn(silu, u);
+    const float a = swiglu(g, u);
     const size_t off = (size_t)r * f + (size_t)b * SI_QK + j;
     if (act) act[off] = a;
     uint16_t dbits;

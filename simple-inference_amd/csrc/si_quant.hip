@@ -242,8 +242,7 @@ __global__ void __launch_bounds__(256) k_swiglu_q8(const float *__restrict__ gu,
     const float *row = gu + (size_t)r * 2 * f;
     const float g = row[b * SI_QK + j];
     const float u = row[f + b * SI_QK + j];
-    const float silu = __fdiv_rn(g, __fadd_rn(1.0f, expf(-g)));
-    const float a = __fmul_rn(silu, u);
+    const float a = swiglu(g, u);
     const size_t off = (size_t)r * f + (size_t)b * SI_QK + j;
     if (act) act[off] = a;
     uint16_t dbits;

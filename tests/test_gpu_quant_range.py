@@ -1,0 +1,72 @@
+"""quantize_q8 and SwiGLU at the ends of their short forms' ranges: block maxima
+around 2^-100 and 2^100 (where the kernels change formulation), zero, subnormal
+and infinite maxima, NaN among the values, ties, against the oracle's bytes."""
+import numpy as np
+import pytest
+
+import si_amd
+from oracle.oracle_py import Oracle
+from tests.gpu_helpers import dev, empty, host, planar_to_aos
+
+pytestmark = pytest.mark.gpu
+QK = 32
+
+MAXIMA = [0.0, 1e-45, 1e-40, 3e-39, 4.3e-37, 1e-36, 1e-31, 2.0 ** -100, 2.0 ** -99.9, 1e-20, 1.0,
+          127.0, 65504.0, 8.4e6, 2.0 ** 99.9, 2.0 ** 100, 1e31, 3.4e38, np.inf]
+
+
+@pytest.mark.parametrize("neighbour", [-1, 0, 1])
+def test_quantize_range_edges(neighbour):
+    rng = np.random.default_rng(11 + neighbour)
+    blocks = []
+    for m in MAXIMA:
+        m = np.float32(m)
+        if neighbour and 0 < m < np.inf:
+            m = np.nextafter(m, np.float32(np.inf if neighbour > 0 else 0), dtype=np.float32)
+        with np.errstate(all="ignore"):
+            x = (rng.uniform(-1, 1, (4, QK)) * m).astype(np.float32)
+            x[1] = (np.arange(QK) - 15.5) * (m / np.float32(127))  # ties
+            x[2, ::5] = np.nan
+            x[3] = 0
+        x[:, 7] = m
+        x[0, 9] = -m
+        blocks.append(x)
+    x = np.concatenate(blocks).astype(np.float32)
+    want = Oracle().quantize_q8(x.reshape(-1))
+    n = x.size
+    import torch
+    tq, td, ts = (empty((k,), t) for k, t in ((n, torch.int8), (n // QK, torch.int16),
+                                              (n // QK, torch.int16)))
+    si_amd.call("si_quantize_q8_rows", si_amd.ptr(dev(x)), 1, n, si_amd.ptr(tq), si_amd.ptr(td),
+                si_amd.ptr(ts), si_amd.stream_handle())
+    qs, d, s = host(tq), host(td).view(np.uint16), host(ts)
+    got = planar_to_aos(qs, d)
+    bad = [i for i in range(len(want)) if got[i].tobytes() != want[i].tobytes()]
+    assert not bad, [(i // 4, i % 4, got[i], want[i]) for i in bad[:3]]
+    assert np.array_equal(s, qs.reshape(-1, QK).astype(np.int32).sum(1).astype(np.int16))
+
+
+def test_swiglu_range_edges():
+    """Against 64 bits, g from where e^-g vanishes to where it overflows; silu's float rounding
+    steps (e^-g, 1 + e^-g, the quotient, the product) bound the error by 4 * 2^-24 relative."""
+    import torch
+    f = 4096
+    g = np.concatenate([np.linspace(-87, 110, f - 8), [0.0, 1e-40, -1e-30, 88.8, 104, 1e30, -60,
+                                                       -86.9]]).astype(np.float32)
+    u = np.random.default_rng(3).normal(0, 1, f).astype(np.float32)
+    act, qs, d = empty((f,), torch.float32), empty((f,), torch.int8), empty((f // QK,), torch.int16)
+    si_amd.call("si_swiglu_q8", si_amd.ptr(dev(np.concatenate([g, u]))), 1, f, si_amd.ptr(act),
+                si_amd.ptr(qs), si_amd.ptr(d), None, si_amd.stream_handle())
+    got = host(act).astype(np.float64)
+    g64 = g.astype(np.float64)
+    with np.errstate(over="ignore"):
+        want = g64 / (1 + np.exp(-g64)) * u
+    assert (np.abs(got - want) <= 4 * 2.0 ** -24 * np.abs(want) + 1e-44).all()
+    # e^-g overflows: the quotient is a zero, an infinite g keeps its value, NaN stays NaN
+    edge = np.array([-89, -1000, -np.inf, np.inf, np.nan] + [0.0] * 27, np.float32)
+    si_amd.call("si_swiglu_q8", si_amd.ptr(dev(np.concatenate([edge, np.ones(QK, np.float32)]))),
+                1, QK, si_amd.ptr(act), si_amd.ptr(qs), si_amd.ptr(d), None,
+                si_amd.stream_handle())
+    got = host(act)[:5]
+    assert got[0] == 0 and got[1] == 0 and np.isnan(got[2]) and got[3] == np.inf and \
+        np.isnan(got[4])
