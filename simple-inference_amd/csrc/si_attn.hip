@@ -392,24 +392,39 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
 // ===========================================================================
 // Causal prefill attention (flash attention over 32 x 32 tiles).
 //
-// One workgroup owns one KV group, 32 consecutive query tokens and NW of
-// the group's query heads (blockIdx.z picks which NW); wavefront w computes
-// one head for those tokens, so each K/V tile staged in LDS serves NW heads.
-// Fewer heads per workgroup give more, shorter workgroups where the tokens
-// alone would not fill the CUs.  Per 32-position K/V tile a
-// wavefront computes
-//     S^T[pos][tok] = K[pos][:] . Q[tok][:]          (v_mfma_f32_32x32x16_f16)
+// The query rows of a KV group are its (token, head) pairs, token-major: row
+// r is head r % per of token r / per (per = qheads / kvheads).  A wavefront
+// computes 32 consecutive rows, so any group size fills its 32 columns (one
+// wavefront per head had left one of eight idle at 7 heads).  A workgroup is
+// RT * KW wavefronts: RT row tiles that share each K/V tile staged in LDS,
+// times KW wavefronts that take every KW-th 32-position tile of the range.
+// The KW states of a row tile meet in LDS at the end, so a long range is
+// walked by several wavefronts at once, with no partials in memory and no
+// merge launch.  Per tile a wavefront computes
+//     S^T[pos][row] = K[pos][:] . Q[row][:]          (v_mfma_f32_32x32x16_f16)
 // (Q split into fp16 hi + lo halves, each product done twice, for fp32-level
-// scores), applies the causal mask and the online softmax per token (a
-// token's 32 scores sit in one lane and its partner lane ^ 32), then
-//     O^T[d][tok] += V^T[d][pos] . P^T[pos][tok]     (v_mfma_f32_32x32x16_f16)
-// The running max and sum of a token then live in the lanes that hold its O^T
-// column, so the rescale is a per-lane multiply.  P is split into fp16 hi +
-// lo halves like Q (an fp16-only P moves outputs by ~1e-3 relative, enough
-// to break the prefill == sequential decode agreement the reference tests).
-// V is staged transposed so the A operand of the PV product is two 8-byte
-// LDS reads per lane.  The epilogue normalises, stores fp32 and quantizes
-// every 32-dim block to Q8_0 (qwen_one_layer.c:272) in registers.
+// scores), the causal mask where the tile reaches a row's position, the online
+// softmax per row in powers of two (a row's 32 scores sit in one lane and its
+// partner lane ^ 32), then
+//     O^T[d][row] += V^T[d][pos] . P^T[pos][row]     (v_mfma_f32_32x32x16_f16)
+// The running max and sum of a row then live in the lanes that hold its O^T
+// column, so the rescale is a per-lane multiply, and rare (below).  P is split into fp16 hi + lo halves like Q (an fp16-only P moves
+// outputs by ~1e-3 relative, enough to break the prefill == sequential decode
+// agreement the reference tests).
+//
+// Bound: the matrix pipe, 2 * (D/16 + D/16) instructions of ~33 cycles per
+// tile (1056 at D = 128) against ~115 VALU operations, 16 of them
+// exponentials (~620 cycles), which two wavefronts per SIMD overlap in part: a
+// tile takes a SIMD about 1600 cycles, a workgroup's first loads and its
+// merge another 8 us.  (Issuing the next tile's scores, or the previous
+// tile's weighing, among the exponentials within a wavefront changed nothing:
+// 92 and 88 us against 87 at 7B x 2048; the second wavefront already fills
+// those gaps.  What helped was fewer VALU operations: 87 -> 77 us.)  K and V tiles are
+// copied global -> LDS by buffer loads that write LDS (no staging registers,
+// no transposition: V^T operands come from the transposing LDS read), their
+// 16-byte chunks permuted within each row on the way so that neither the
+// score operands (32 rows, one chunk) nor the transposing reads (4 rows, 4
+// chunks) meet in a bank.
 //
 // 32x32 layouts: output (i, j) is held by lane j + 32*((i/4)%2), register
 // (i%4) + 4*(i/8); operand lane l supplies row (or column) l%32 and k-slice
@@ -417,269 +432,365 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
 // reduction indices to (slice, element) is exact.
 // ===========================================================================
 typedef float f16v __attribute__((ext_vector_type(16)));
-typedef int pf_v4i __attribute__((ext_vector_type(4)));
+typedef _Float16 pf_h2 __attribute__((ext_vector_type(2)));
+typedef float pf_f2 __attribute__((ext_vector_type(2)));
 
-constexpr int PF_T = 32;      // query tokens per workgroup, positions per K/V tile
-constexpr int PF_KPAD = 8;    // halves of padding per K row
-constexpr int PF_VPAD = 4;    // halves of padding per V^T row (18-dword rows)
+constexpr int PF_T = 32;      // query rows per wavefront, positions per K/V tile
+constexpr int PF_OPAD = 4;    // floats of padding per merged output row
 
-// Causal balance: query tiles qsplit..nqt-1 (nsplit of them) run as two
-// workgroups each, over K/V tiles [0, cap) and [cap, end); their partial
-// states go to ws_* as [token - 32*qsplit][head][2] and k_attn_combine
-// merges them.
-struct PrefillSplit {
-    int nqt, qsplit, nsplit, cap;
-    float *ws_m, *ws_l, *ws_o;
-};
+// LDS slot (16-byte unit within the row) of chunk c of tile row r: the 16
+// rows a score operand read takes together, and the 4 rows x 4 chunks of a
+// transposing read, spread over the 64 banks
+template <int D>
+__device__ __forceinline__ int pf_k_slot(int r, int c) {
+    if (D == 128) return c ^ (r & 15);
+    if (D == 64) return c ^ ((r >> 1) & 7);
+    if (D == 32) return c ^ ((r >> 2) & 3);
+    const int s = c + ((r >> 2) & 3);  // 12 chunks: a rotation
+    return s >= D / 8 ? s - D / 8 : s;
+}
+template <int D>
+__device__ __forceinline__ int pf_v_slot(int r, int c) {
+    if (D == 128) return c ^ ((r & 3) << 2);
+    if (D == 64) return c ^ (((r >> 1) & 1) << 2);
+    return c;  // 4 rows already cover the banks
+}
+// the chunk whose slot is s
+template <int D>
+__device__ __forceinline__ int pf_k_chunk(int r, int s) {
+    if (D != 96) return pf_k_slot<D>(r, s);  // an XOR
+    const int c = s - ((r >> 2) & 3);
+    return c < 0 ? c + D / 8 : c;
+}
 
-template <int D, int NW>
-struct PrefillLds {
-    static constexpr int KROW = D + PF_KPAD, VROW = PF_T + PF_VPAD;
-    static constexpr size_t bytes() { return (size_t)(PF_T * KROW + D * VROW) * 2; }
-};
+// (fmaxf of matrix results would first canonicalise each; a must come from an
+// ordinary operation on those results)
+__device__ __forceinline__ float max3_f(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+// two values as fp16 hi + lo halves (hi rounded to nearest, lo = x - hi by a
+// mixed-precision fma; the plain conversion to hi reads both values first)
+__device__ __forceinline__ void split_pair(float x0, float x1, pf_h2 &hi, pf_h2 &lo) {
+    hi = __builtin_convertvector((pf_f2){x0, x1}, pf_h2);
+    float l0, l1;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(l0) : "v"(hi), "v"(x0));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+        : "=v"(l1)
+        : "v"(hi), "v"(x1));
+    lo = __builtin_convertvector((pf_f2){l0, l1}, pf_h2);
+}
 
-template <int D, int NW>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) k_attn_prefill(
-    const float *__restrict__ q, int ntok, int qheads, int kvheads, int pos0,
-    const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc, float scale,
-    float *__restrict__ attn, int8_t *__restrict__ qs, uint16_t *__restrict__ qd,
-    int16_t *__restrict__ bsum, PrefillSplit sp) {
-    using Lds = PrefillLds<D, NW>;
-    constexpr int NT = NW * 64, KS = D / 16, DT = D / 32;
-    constexpr int KPIECES = PF_T * D / 8;        // 16-byte K pieces per tile
-    constexpr int VITEMS = (PF_T / 2) * (D / 8); // (position pair, 8 dims) per tile
-    constexpr int KPT = (KPIECES + NT - 1) / NT, VPT = (VITEMS + NT - 1) / NT;
-    extern __shared__ __attribute__((aligned(16))) uint8_t pf_sm[];
-    _Float16 *k_l = (_Float16 *)pf_sm;                  // [PF_T][KROW]
-    _Float16 *vt_l = k_l + PF_T * Lds::KROW;            // [D][VROW]
+// at most VM vector-memory operations of this wavefront outstanding, its LDS
+// reads complete
+template <int VM>
+__device__ __forceinline__ void pf_wait() {
+    static_assert(VM <= 63, "vmcnt holds 6 bits");
+    __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4));
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void pf_barrier() {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
 
-    // work unit of this workgroup, longest first: the first K/V halves of
-    // the split query tiles, then their second halves interleaved with the
-    // unsplit tiles (unit -1: whole range, 0: [0, cap), 1: [cap, end)).
-    // Odd head subsets take the units in reverse order: the workgroups that
-    // share a CU (dispatched a whole subset apart) then pair a long query
-    // tile with a short one (7B, 2048 tokens: 150 -> 118 us).
-    int qt, unit;
-    {
-        const int b = (blockIdx.z & 1) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
-        const int S = sp.nsplit, Q0 = sp.qsplit;
-        if (b < S) {
-            qt = sp.nqt - 1 - b;
-            unit = 0;
-        } else {
-            const int bp = b - S, m2 = min(S, Q0);
-            if (bp < 2 * m2) {
-                const int k = bp >> 1;
-                qt = (bp & 1) ? Q0 - 1 - k : sp.nqt - 1 - k;
-                unit = (bp & 1) ? -1 : 1;
-            } else {
-                const int r = m2 + (bp - 2 * m2);
-                qt = S > Q0 ? sp.nqt - 1 - r : Q0 - 1 - r;
-                unit = S > Q0 ? 1 : -1;
-            }
-        }
-    }
-    const int g = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+template <int D, int RT, int KW>
+__global__ void __launch_bounds__(RT * KW * 64) __attribute__((amdgpu_waves_per_eu(2)))
+k_attn_prefill(const float *__restrict__ q, int ntok, int qheads, int kvheads, int pos0,
+               const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc, float scale2,
+               float *__restrict__ attn, int8_t *__restrict__ qs, uint16_t *__restrict__ qd,
+               int16_t *__restrict__ bsum) {
+    constexpr int NWV = RT * KW, NT = NWV * 64, KS = D / 16, DT = D / 32, CH = D / 8;
+    constexpr int TB = PF_T * D * 2;            // bytes of a K (or V) tile
+    constexpr int TI = TB / 1024;               // copy instructions per tile
+    constexpr int TIW = (TI + RT - 1) / RT;     // of one wavefront
+    constexpr int OROW = D + PF_OPAD;
+    // RT > 1: two stage buffers (K tiles, then V tiles) used in turn, one
+    // barrier per step.  RT == 1: each wavefront stages its own tiles, K in
+    // sb0 and V in sb1, each refilled as soon as it has been read (no
+    // barrier).  At the end the wavefronts' outputs: the first half in sb0,
+    // the others in sb1.
+    constexpr bool DB = RT > 1;
+    constexpr int STAGE = DB ? 2 * KW * TB : KW * TB;
+    constexpr int HALF_W = (NWV + 1) / 2, MRG = HALF_W * PF_T * OROW * 4;
+    __shared__ __attribute__((aligned(16))) uint8_t sb0[STAGE > MRG ? STAGE : MRG];
+    __shared__ __attribute__((aligned(16))) uint8_t sb1[STAGE > MRG ? STAGE : MRG];
+    __shared__ float mrg_m[NWV][PF_T], mrg_l[NWV][PF_T];
+    __shared__ int64_t rowoff[32 * RT];  // output offset of a row, -1 past the last
+
+    const int per = qheads / kvheads, nrows = ntok * per;
+    const int units = (nrows + 32 * RT - 1) / (32 * RT);
+    // workgroups of one KV group go to the same XCDs (id % 8) where the group
+    // count divides 8; the longest ranges first
+    const int g = blockIdx.x % kvheads, unit = units - 1 - blockIdx.x / kvheads;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kw = wave / RT, rt = wave % RT;
     const int t = lane & 31, hh = lane >> 5;
-    const int per = qheads / kvheads;
-    const int hw = blockIdx.z * NW + w;  // head within the group
-    const bool active = hw < per;
-    const int h = g * per + (active ? hw : 0);
-    const int tq = qt * PF_T + t;  // this lane's query token
-    const int ptq = pos0 + tq;     // its position: it sees cache rows 0..ptq
     const int kvd = kvheads * D;
-    const int last = min(pos0 + qt * PF_T + PF_T - 1, pos0 + ntok - 1);  // last cache row used
-    const int it0 = unit == 1 ? sp.cap : 0;
-    const int it1 = unit == 0 ? sp.cap : last / PF_T + 1;
+    const int r0 = unit * 32 * RT;  // the workgroup's first row
+    const int wr0 = r0 + 32 * rt;   // this wavefront's
+    // last cache rows of the workgroup and of this wavefront's tile
+    const int last = pos0 + min(r0 + 32 * RT - 1, nrows - 1) / per;
+    const int wlast = pos0 + min(wr0 + 31, nrows - 1) / per;
+    const int wfirst = pos0 + min(wr0, nrows - 1) / per;  // its lowest causal limit
+    const int steps = last / (PF_T * KW) + 1;
+    const int myrow = min(wr0 + t, nrows - 1);
+    const int prow = pos0 + myrow / per;  // the row's position: it sees cache rows 0..prow
 
-    // Q^T as the B operand of the score MFMA: column tok = t, k-slice hh
+    // this wavefront's copies of a tile: instruction i takes the 16-byte
+    // units 64 i .. 64 i + 63 of the tile (LDS order)
+    int crow[TIW], ck[TIW], cv[TIW];
+#pragma unroll
+    for (int i = 0; i < TIW; ++i) {
+        const int p = (rt + RT * i) * 64 + lane;
+        const int row = p / CH, slot = p % CH;
+        crow[i] = row;
+        ck[i] = pf_k_chunk<D>(row, slot) * 16;
+        cv[i] = pf_v_slot<D>(row, slot) * 16;  // its own inverse
+    }
+    const auto copy = [&](const uint16_t *base, uint8_t *dst, int step, const int (&col)[TIW]) {
+        const int kv0 = min(step * KW + kw, last / PF_T) * PF_T;  // past the range: the last tile
+        const __amdgpu_buffer_rsrc_t rs = buf_rsrc(base + (size_t)kv0 * kvd + g * D, 0x7fffffffu);
+#pragma unroll
+        for (int i = 0; i < TIW; ++i)
+            if (TI % RT == 0 || rt + RT * i < TI)
+                // rows past the last one read it again (masked out)
+                lds_copy16(rs, dst + kw * TB + 1024 * (rt + RT * i),
+                           (uint32_t)(min(crow[i], last - kv0) * (kvd * 2) + col[i]));
+    };
+    copy(kc, sb0, 0, ck);
+    copy(vc, DB ? sb0 + KW * TB : sb1, 0, cv);
+
+    // Q^T as the B operand of the score MFMA: column t, k-slice hh (columns
+    // past the last row repeat it and are never stored)
+    const size_t qoff = ((size_t)(myrow / per) * qheads + g * per + myrow % per) * D;
+    if (kw == 0 && hh == 0) rowoff[32 * rt + t] = wr0 + t < nrows ? (int64_t)qoff : -1;
     h8 qh[KS], ql[KS];
     {
-        const bool ok = active && tq < ntok;
-        const float *qrow = q + ((size_t)(ok ? tq : 0) * qheads + h) * D;
+        const float *qrow = q + qoff + 8 * hh;
+        float4 a[KS], b[KS];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            const float4 a = *(const float4 *)(qrow + 16 * ks + 8 * hh);
-            const float4 b = *(const float4 *)(qrow + 16 * ks + 8 * hh + 4);
-            const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            a[ks] = *(const float4 *)(qrow + 16 * ks);
+            b[ks] = *(const float4 *)(qrow + 16 * ks + 4);
+        }
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                _Float16 hi, lo;
-                split_hi_lo(ok ? x[e] : 0.0f, hi, lo);
-                qh[ks][e] = hi;
-                ql[ks][e] = lo;
+        for (int ks = 0; ks < KS; ++ks) {
+            const float x[8] = {a[ks].x, a[ks].y, a[ks].z, a[ks].w,
+                                b[ks].x, b[ks].y, b[ks].z, b[ks].w};
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                pf_h2 hi, lo;
+                split_pair(x[e], x[e + 1], hi, lo);
+                qh[ks][e] = hi[0];
+                qh[ks][e + 1] = hi[1];
+                ql[ks][e] = lo[0];
+                ql[ks][e + 1] = lo[1];
             }
         }
     }
 
-    // register staging of one K/V tile (rows clamped to `last`; the clamped
-    // duplicates lie past every token's causal limit and are masked)
-    // clang vectors, not uint4 structs: arrays of those stay in registers
-    pf_v4i rk[KPT], rv[VPT][2];
-    auto load_tile = [&](int kv0) {
+    // operand addresses within a stage: K row t, chunk 2 ks + hh; V rows
+    // 16 s2 + 8 e + 4 hh + s / 4 (s = lane % 16), columns 32 dt + 16 (lane /
+    // 16 % 2) + 4 (s % 4), as the transposing read takes them
+    const int s16 = lane & 15;
+    int ka[KS], va[DT];
 #pragma unroll
-        for (int i = 0; i < KPT; ++i) {
-            const int c = min(tid + NT * i, KPIECES - 1);
-            const int r = c / (D / 8), e8 = c % (D / 8);
-            const int pos = min(kv0 + r, last);
-            rk[i] = *(const pf_v4i *)(kc + (size_t)pos * kvd + (size_t)g * D + 8 * e8);
-        }
+    for (int ks = 0; ks < KS; ++ks) ka[ks] = kw * TB + t * D * 2 + pf_k_slot<D>(t, 2 * ks + hh) * 16;
 #pragma unroll
-        for (int i = 0; i < VPT; ++i) {
-            const int c = min(tid + NT * i, VITEMS - 1);
-            const int pr = c % (PF_T / 2), e8 = c / (PF_T / 2);
-            const int p0 = min(kv0 + 2 * pr, last), p1 = min(kv0 + 2 * pr + 1, last);
-            rv[i][0] = *(const pf_v4i *)(vc + (size_t)p0 * kvd + (size_t)g * D + 8 * e8);
-            rv[i][1] = *(const pf_v4i *)(vc + (size_t)p1 * kvd + (size_t)g * D + 8 * e8);
-        }
-    };
-    auto store_tile = [&]() {
-#pragma unroll
-        for (int i = 0; i < KPT; ++i) {
-            const int c = tid + NT * i;
-            if (KPIECES % NT == 0 || c < KPIECES) {
-                const int r = c / (D / 8), e8 = c % (D / 8);
-                *(pf_v4i *)(k_l + r * Lds::KROW + 8 * e8) = rk[i];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < VPT; ++i) {
-            const int c = tid + NT * i;
-            if (VITEMS % NT == 0 || c < VITEMS) {
-                // position pairs fastest: with 18-dword V^T rows the 64
-                // lanes' 4-byte writes hit 64 distinct banks
-                const int pr = c % (PF_T / 2), e8 = c / (PF_T / 2);
-                const uint32_t a[4] = {(uint32_t)rv[i][0][0], (uint32_t)rv[i][0][1],
-                                       (uint32_t)rv[i][0][2], (uint32_t)rv[i][0][3]};
-                const uint32_t b[4] = {(uint32_t)rv[i][1][0], (uint32_t)rv[i][1][1],
-                                       (uint32_t)rv[i][1][2], (uint32_t)rv[i][1][3]};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    // dims 8*e8 + 2j (low halves) and + 2j + 1 (high halves)
-                    const uint32_t lo = __builtin_amdgcn_perm(b[j], a[j], 0x05040100u);
-                    const uint32_t hi = __builtin_amdgcn_perm(b[j], a[j], 0x07060302u);
-                    *(uint32_t *)(vt_l + (8 * e8 + 2 * j) * Lds::VROW + 2 * pr) = lo;
-                    *(uint32_t *)(vt_l + (8 * e8 + 2 * j + 1) * Lds::VROW + 2 * pr) = hi;
-                }
-            }
-        }
-    };
+    for (int dt = 0; dt < DT; ++dt)
+        va[dt] = kw * TB + (4 * hh + (s16 >> 2)) * D * 2 +
+                 pf_v_slot<D>(s16 >> 2, 4 * dt + 2 * ((lane >> 4) & 1) + ((s16 & 3) >> 1)) * 16 +
+                 (s16 & 1) * 8;
 
-    float m = -INFINITY, lsum = 0.0f;  // softmax state of token t (same in both halves)
+    float m = -INFINITY, lsum = 0.0f;  // row t's running max; this lane's share of the sum
     f16v o[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) o[dt] = (f16v){};
 
-    load_tile(it0 * PF_T);
-    for (int it = it0; it < it1; ++it) {
-        const int kv0 = it * PF_T;
-        store_tile();
-        __syncthreads();
-        // next tile in flight, unconditionally (the last iteration re-reads
-        // its own rows): a conditional load keeps the staging registers in
-        // scratch memory and waits for every load
-        load_tile(min(kv0 + PF_T, (it1 - 1) * PF_T));
-        if (active) {
-            // scores S^T[pos = kv0 + i][tok = t]
-            f16v sh = (f16v){}, sl = (f16v){};  // two independent MFMA chains
-            const _Float16 *krow = k_l + t * Lds::KROW + 8 * hh;  // A row pos = lane % 32
+    const auto load_k = [&](const uint8_t *kt, h8 (&a)[KS]) {
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const h8 ka = *(const h8 *)(krow + 16 * ks);
-                sh = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qh[ks], sh, 0, 0, 0);
-                sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, ql[ks], sl, 0, 0, 0);
-            }
-            const f16v sacc = sh + sl;
-            float sv[16];
-            float mx = -INFINITY;
+        for (int ks = 0; ks < KS; ++ks) a[ks] = *(const h8 *)(kt + ka[ks]);
+    };
+    const auto scores = [&](const h8 (&a)[KS]) {
+        // the lo products first: they round at their own small magnitude
+        f16v s = (f16v){};
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int pos = kv0 + 8 * (r >> 2) + 4 * hh + (r & 3);
-                sv[r] = pos <= ptq ? sacc[r] * scale : -INFINITY;
-                mx = fmaxf(mx, sv[r]);
-            }
-            mx = fmaxf(mx, swap32_f(mx));
-            const float mnew = fmaxf(m, mx);
-            // a second K/V half can be entirely past a token's causal limit:
-            // its state stays (-inf, 0, 0) instead of turning NaN
-            const float mref = mnew == -INFINITY ? 0.0f : mnew;
-            const float alpha = __expf(m - mref);
-            float ps = 0.0f;
-            h8 pbh[2], pbl[2];
+        for (int ks = 0; ks < KS; ++ks)
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks], ql[ks], s, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float pr = __expf(sv[r] - mref);
-                ps += pr;
-                _Float16 hi, lo;
-                split_hi_lo(pr, hi, lo);
-                pbh[r >> 3][r & 7] = hi;
-                pbl[r >> 3][r & 7] = lo;
-            }
-            ps += swap32_f(ps);
-            lsum = fmaf(lsum, alpha, ps);
-            m = mnew;
-            // O^T[d][tok] += V^T[d][pos] P^T[pos][tok]; k-step s2 covers
-            // positions 16*s2 + 8*(e/4) + 4*hh + e%4 (e = element 0..7), the
-            // positions of registers 8*s2 + e of the score output
+        for (int ks = 0; ks < KS; ++ks)
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks], qh[ks], s, 0, 0, 0);
+        return s;
+    };
+    h8 ph[2], pl[2];  // the tile's weights
+    const auto softmax = [&](f16v s, int kv0) {
+        if (kv0 + PF_T - 1 > wfirst) {  // wavefront-uniform: the tile reaches a causal limit
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-                f16v acc = o[dt] * alpha;
-                const _Float16 *vrow = vt_l + (32 * dt + t) * Lds::VROW + 4 * hh;
-#pragma unroll
-                for (int s2 = 0; s2 < 2; ++s2) {
-                    const h4 v0 = *(const h4 *)(vrow + 16 * s2);
-                    const h4 v1 = *(const h4 *)(vrow + 16 * s2 + 8);
-                    const h8 va = (h8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pbh[s2], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pbl[s2], acc, 0, 0, 0);
-                }
-                o[dt] = acc;
-            }
+            for (int r = 0; r < 16; ++r)
+                s[r] = kv0 + 8 * (r >> 2) + 4 * hh + (r & 3) <= prow ? s[r] : -INFINITY;
         }
-        __syncthreads();  // the tile's LDS is rewritten next
+        // (a plain operation reads the matrix results first: the compiler
+        // puts the wait states they need before it, which it would not
+        // before the inline instructions that follow from it)
+        float mx = fmaxf(s[0], s[1]);
+#pragma unroll
+        for (int r = 2; r < 16; r += 2) mx = max3_f(mx, s[r], s[r + 1]);
+        mx = fmaxf(mx, swap32_f(mx));
+        // The weights are taken against m, a max of the row so far (in powers
+        // of two: scale2 * score) that follows the running max only when that
+        // has grown by more than 2^8: weights up to 256 lose nothing, and the
+        // rescale of the sums, which some row of the 32 would otherwise ask
+        // for in most tiles, becomes rare.  A wavefront's first tiles can lie
+        // past a row's limit: its state stays (-inf, 0, 0), no NaN.
+        const float mnew = fmaxf(m, mx * scale2);
+        if (__ballot(mnew > m + 8.0f)) {
+            const float alpha = __builtin_amdgcn_exp2f(m - mnew);
+            const float a0 = mnew == -INFINITY ? 1.0f : alpha;
+            lsum *= a0;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] *= a0;
+            m = mnew;
+        }
+        const float mref = m == -INFINITY ? 0.0f : m;
+        float ps = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(s[r], scale2, -mref));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(s[r + 1], scale2, -mref));
+            ps += p0;
+            ps += p1;
+            pf_h2 hi, lo;
+            split_pair(p0, p1, hi, lo);
+            ph[r >> 3][r & 7] = hi[0];
+            ph[r >> 3][(r & 7) + 1] = hi[1];
+            pl[r >> 3][r & 7] = lo[0];
+            pl[r >> 3][(r & 7) + 1] = lo[1];
+        }
+        lsum += ps;
+    };
+    const auto weigh = [&](const uint8_t *vt) {
+        // k-step s2 covers positions 16*s2 + 8*(e/4) + 4*hh + e%4 (e = element
+        // 0..7), the positions of registers 8*s2 + e of the score output
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2) {
+                const h4 v0 = __builtin_bit_cast(h4, lds_read_tr16(vt + va[dt] + 16 * s2 * D * 2));
+                const h4 v1 =
+                    __builtin_bit_cast(h4, lds_read_tr16(vt + va[dt] + (16 * s2 + 8) * D * 2));
+                const h8 a = (h8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph[s2], o[dt], 0, 0, 0);
+                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl[s2], o[dt], 0, 0, 0);
+            }
+    };
+    if constexpr (DB) {
+        // one step: the stage is complete and the other buffer free after the
+        // barrier; the next stage's copies run during the whole step
+        const auto step = [&](uint8_t *cur, uint8_t *nxt, int st) {
+            pf_wait<0>();
+            pf_barrier();
+            if (st + 1 < steps) {
+                copy(kc, nxt, st + 1, ck);
+                copy(vc, nxt + KW * TB, st + 1, cv);
+            }
+            const int kv0 = (st * KW + kw) * PF_T;
+            if (kv0 <= wlast) {  // wavefront-uniform
+                h8 a[KS];
+                load_k(cur, a);
+                softmax(scores(a), kv0);
+                weigh(cur + KW * TB);
+            }
+        };
+        for (int st = 0; st < steps; st += 2) {
+            step(sb0, sb1, st);
+            if (st + 1 < steps) step(sb1, sb0, st + 1);
+        }
+    } else {
+        for (int st = 0; st < steps; ++st) {
+            const int kv0 = (st * KW + kw) * PF_T;
+            if (kv0 > wlast) break;  // wavefront-uniform
+            const bool more = kv0 + KW * PF_T <= wlast;
+            pf_wait<TIW>();  // K is in; V may still be on its way
+            h8 a[KS];
+            load_k(sb0, a);
+            pf_wait<TIW>();  // K has been read
+            if (more) copy(kc, sb0, st + 1, ck);
+            softmax(scores(a), kv0);
+            if (more)
+                pf_wait<TIW>();  // V is in; the next K may still be on its way
+            else
+                pf_wait<0>();
+            weigh(sb1);
+            pf_wait<TIW>();  // V has been read
+            if (more) copy(vc, sb1, st + 1, cv);
+        }
     }
+    lsum += swap32_f(lsum);
+    pf_wait<0>();  // no copy in flight (a wavefront without tiles never waited for its own)
+    __syncthreads();  // every wavefront is done with the stage buffers
 
-    if (!active || tq >= ntok) return;
-    // lane holds O[tok][32*dt + 8*(r/4) + 4*hh + r%4] in o[dt][r]
-    if (unit >= 0) {  // a half of a split tile: (max, sum, unnormalised O) for the merge
-        const size_t pi = ((size_t)(tq - sp.qsplit * PF_T) * qheads + h) * 2 + unit;
+    // lane (t, hh) holds O[row t][32*dt + 8*(r/4) + 4*hh + r%4] in o[dt][r]
+    {
+        float *mo = (float *)(wave < HALF_W ? sb0 : sb1) + (wave % HALF_W) * (PF_T * OROW);
         if (hh == 0) {
-            sp.ws_m[pi] = m;
-            sp.ws_l[pi] = lsum;
+            mrg_m[wave][t] = m;
+            mrg_l[wave][t] = lsum;
         }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4)
-                *(float4 *)(sp.ws_o + pi * D + 32 * dt + 8 * r4 + 4 * hh) =
-                    make_float4(o[dt][4 * r4], o[dt][4 * r4 + 1], o[dt][4 * r4 + 2],
-                                o[dt][4 * r4 + 3]);
-        return;
+                *(f4 *)(mo + t * OROW + 32 * dt + 8 * r4 + 4 * hh) =
+                    (f4){o[dt][4 * r4], o[dt][4 * r4 + 1], o[dt][4 * r4 + 2], o[dt][4 * r4 + 3]};
     }
-    const float inv = 1.0f / lsum;
-    const size_t rowoff = ((size_t)tq * qheads + h) * D;
+    __syncthreads();
+    // a row's factors for its KW states: 2^(m_k - max) / sum, in mrg_m
+    if (tid < 32 * RT) {
+        const int w0 = tid >> 5, tr = tid & 31;
+        float M = -INFINITY, l = 0.0f, f[KW];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-        float y[16];
+        for (int k = 0; k < KW; ++k) M = fmaxf(M, mrg_m[k * RT + w0][tr]);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) y[r] = o[dt][r] * inv;
+        for (int k = 0; k < KW; ++k) {
+            f[k] = __builtin_amdgcn_exp2f(mrg_m[k * RT + w0][tr] - M);
+            l = fmaf(mrg_l[k * RT + w0][tr], f[k], l);
+        }
+        const float inv = 1.0f / l;
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4)
-            *(float4 *)(attn + rowoff + 32 * dt + 8 * r4 + 4 * hh) =
-                make_float4(y[4 * r4], y[4 * r4 + 1], y[4 * r4 + 2], y[4 * r4 + 3]);
+        for (int k = 0; k < KW; ++k) mrg_m[k * RT + w0][tr] = f[k] * inv;
+    }
+    __syncthreads();
+    // 4 consecutive elements of a row per thread: merge the KW states,
+    // quantize (8 lanes hold one Q8_0 block, qwen_one_layer.c:272)
+    constexpr int EL = 32 * RT * D / 4;
+    static_assert(EL % NT == 0, "whole rounds");
+#pragma unroll 2
+    for (int e = tid; e < EL; e += NT) {
+        const int lr = e / (D / 4), dd = 4 * (e % (D / 4)), w0 = lr >> 5, tr = lr & 31;
+        float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+            const int w = k * RT + w0;
+            const float *mo = (const float *)(w < HALF_W ? sb0 : sb1) + (w % HALF_W) * (PF_T * OROW);
+            const f4 v = *(const f4 *)(mo + tr * OROW + dd);
+            const float f = mrg_m[w][tr];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = fmaf(v[i], f, y[i]);
+        }
+        uint16_t dbits;
+        int sum;
+        const uint32_t packed = quant_block_oct(y, dbits, sum);  // every lane of the group
+        if (rowoff[lr] < 0) continue;  // whole 8-lane groups
+        const size_t off = (size_t)rowoff[lr] + dd;
+        *(float4 *)(attn + off) = make_float4(y[0], y[1], y[2], y[3]);
         if (qs) {
-            uint32_t qv[4];
-            uint16_t dbits;
-            int sum;
-            quant_block_pair16(y, qv, dbits, sum);
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4)
-                *(uint32_t *)(qs + rowoff + 32 * dt + 8 * r4 + 4 * hh) = qv[r4];
-            if (hh == 0) {
-                const size_t bi = (rowoff + 32 * dt) / SI_QK;
-                qd[bi] = dbits;
-                if (bsum) bsum[bi] = (int16_t)sum;
+            *(uint32_t *)(qs + off) = packed;
+            if ((tid & 7) == 0) {
+                qd[off / SI_QK] = dbits;
+                if (bsum) bsum[off / SI_QK] = (int16_t)sum;
             }
         }
     }
@@ -692,84 +803,59 @@ bool attn_prefill_supported(int qheads, int kvheads, int hdim) {
            (hdim == 32 || hdim == 64 || hdim == 96 || hdim == 128);
 }
 
-// Split plan of a causal prefill: when the tiles do not fill the CUs, a
-// query tile whose K/V range exceeds half of the longest one is cut in two
-// (more workgroups, each at most half the longest range).  A grid that
-// already fills the chip is not split: measured at 7B / 2048 tokens (256
-// workgroups), the split ran slower (164 + 19 us merge vs 148 us).
-static PrefillSplit prefill_split(int ntok, int pos0, int kvheads) {
-    PrefillSplit p{};
-    p.nqt = (ntok + PF_T - 1) / PF_T;
-    auto tiles = [&](int qt) { return min(pos0 + qt * PF_T + PF_T - 1, pos0 + ntok - 1) / PF_T + 1; };
-    const int longest = tiles(p.nqt - 1);
-    p.cap = (longest + 1) / 2;
-    p.qsplit = p.nqt;
-    if (longest >= 4 && p.nqt * kvheads < 256)  // short ranges or a full grid: unsplit
-        while (p.qsplit > 0 && tiles(p.qsplit - 1) > p.cap) --p.qsplit;
-    p.nsplit = p.nqt - p.qsplit;
-    return p;
-}
-
+// What si_attention_workspace states for a causal prefill: callers size (and
+// si_attention_static accepts or refuses) by it.  The kernel itself merges
+// in LDS and uses none.
 size_t attn_prefill_workspace_bytes(int qheads, int hdim, int ntok) {
     return (size_t)ntok * qheads * 2 * (hdim + 2) * sizeof(float);
 }
 
 void launch_attn_prefill(const float *q, int ntok, int qheads, int kvheads, int hdim, int pos0,
                          const uint16_t *kc, const uint16_t *vc, float *attn, int8_t *qs,
-                         uint16_t *qd, int16_t *bsum, void *workspace, size_t ws_bytes,
-                         hipStream_t st) {
+                         uint16_t *qd, int16_t *bsum, hipStream_t st) {
     if (ntok <= 0) return;
     const int per = qheads / kvheads;
-    PrefillSplit sp = prefill_split(ntok, pos0, kvheads);
-    const int rows_split = ntok - sp.qsplit * PF_T;
-    if (sp.nsplit > 0 &&
-        (!workspace || ws_bytes < attn_prefill_workspace_bytes(qheads, hdim, rows_split))) {
-        sp.qsplit = sp.nqt;  // no room for the partial states: unsplit
-        sp.nsplit = 0;
-    }
-    if (sp.nsplit > 0) {
-        const size_t np = (size_t)rows_split * qheads * 2;
-        sp.ws_m = (float *)workspace;
-        sp.ws_l = sp.ws_m + np;
-        sp.ws_o = sp.ws_l + np;
-    }
-    // heads per workgroup: up to 8 (a wider group takes several
-    // workgroups), halved while the grid has fewer than ~2 workgroups per CU
-    // (down to 2 heads for hdim >= 96, whose one-wavefront workgroups would
-    // spill registers)
-    const int units = 2 * sp.nsplit + sp.qsplit;
-    const int nw_min = hdim >= 96 ? 2 : 1;
-    int nw = 8;
-    while (nw > nw_min && (size_t)units * kvheads * ((per + nw - 1) / nw) < 512) nw /= 2;
-    const dim3 grid(units, kvheads, (per + nw - 1) / nw);
-    const float scale = 1.0f / sqrtf((float)hdim);  // attention_kernels.h:86
-#define PF_CALL(DIM, NW)                                                                      \
-    SI_LAUNCH((k_attn_prefill<DIM, NW>), grid, dim3(NW * 64),                                 \
-              (PrefillLds<DIM, NW>::bytes()), st, q, ntok, qheads, kvheads, pos0, kc,         \
-              vc, scale, attn, qs, qd, bsum, sp)
-#define PF_DIM(DIM)                     \
-    switch (nw) {                       \
-        case 1: PF_CALL(DIM, 1); break; \
-        case 2: PF_CALL(DIM, 2); break; \
-        case 4: PF_CALL(DIM, 4); break; \
-        default: PF_CALL(DIM, 8);       \
+    // scores in powers of two: exp(s / sqrt(hdim)) (attention_kernels.h:86)
+    const float scale2 = 1.44269504088896340736f / sqrtf((float)hdim);
+    // Wavefronts per workgroup, by the number of 32-row tiles.  While they are
+    // fewer than two per CU each tile gets a workgroup of its own, its range
+    // walked four ways; past that two or four tiles share each staged K/V
+    // tile, two ways.  Measured (us, kernel alone; RT x KW = 1x4, 2x2, 4x2;
+    // before: one wavefront per head and tokens, the range split in memory):
+    //   0.5B 512 tokens (224 tiles)          7.9   10.5   13.0   before 17.2
+    //   7B 333 after 1500 (292)             32.3   39.0   50.0          71.2
+    //   7B 512 (448)                        15.2   17.6   21.7          31.1
+    //   7B 700 after 2000 (616)             80.6   70.3   73.9         113
+    //   0.5B 2048 (896)                     26.7   31.0   36.6          59.8
+    //   0.5B 4000 (1750)                    77.3   72.8   77.8         144
+    //   7B 2048 (1792)                      93.7   81.1   76.8         110
+    //   12 heads of 128, 5000 (1876)         186    173    157         315
+    const long rows = (long)ntok * per;
+    const long tiles = (rows + 31) / 32 * kvheads;
+    const int rt = tiles < (hdim <= 64 ? 1024 : 512) ? 1 : hdim <= 64 || tiles < 1280 ? 2 : 4;
+    const dim3 grid((unsigned)((rows + 32 * rt - 1) / (32 * rt) * kvheads));
+#define PF_CALL(DIM, RT, KW)                                                                 \
+    SI_LAUNCH((k_attn_prefill<DIM, RT, KW>), grid, dim3(RT * KW * 64), 0, st, q, ntok, qheads, \
+              kvheads, pos0, kc, vc, scale2, attn, qs, qd, bsum)
+#define PF_DIM(DIM)                        \
+    switch (rt) {                          \
+        case 1: PF_CALL(DIM, 1, 4); break; \
+        default: PF_CALL(DIM, 2, 2);       \
     }
     switch (hdim) {
         case 32: PF_DIM(32); break;
         case 64: PF_DIM(64); break;
-        case 96: PF_DIM(96); break;
-        default: PF_DIM(128); break;
+        case 96:
+            if (rt == 4) PF_CALL(96, 4, 2);
+            else PF_DIM(96);
+            break;
+        default:
+            if (rt == 4) PF_CALL(128, 4, 2);
+            else PF_DIM(128);
+            break;
     }
 #undef PF_DIM
 #undef PF_CALL
-    if (sp.nsplit > 0) {
-        const size_t t0 = (size_t)sp.qsplit * PF_T, qd_ = (size_t)qheads * hdim;
-        SI_LAUNCH(k_attn_combine, dim3(qheads, rows_split), dim3(hdim), 0, st, qheads,
-                  hdim, 2, sp.ws_m, sp.ws_l, sp.ws_o, attn + t0 * qd_,
-                  qs ? qs + t0 * qd_ : nullptr, qs ? qd + t0 * qd_ / SI_QK : nullptr,
-                  bsum ? bsum + t0 * qd_ / SI_QK : nullptr, (int8_t *)nullptr,
-                  (uint16_t *)nullptr);
-    }
 }
 
 // Context chunks per (query, KV group): enough workgroups to cover the chip

@@ -576,18 +576,6 @@ __device__ __forceinline__ v8i f6_operand(const uint8_t *p16, const uint8_t *p8)
     return (v8i){(int)a.x, (int)a.y, (int)a.z, (int)a.w, (int)b.x, (int)b.y, 0, 0};
 }
 
-typedef __attribute__((address_space(3))) void lds_void;
-
-// One wavefront copy global -> LDS: lane l's 16 bytes at voff of r land at
-// lds + 16 l; a 2-byte copy lands zero-extended in the dword at lds + 4 l
-// (measured on MI355X); lds wavefront-uniform.
-__device__ __forceinline__ void lds_copy16(__amdgpu_buffer_rsrc_t r, uint8_t *lds, uint32_t voff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 16, voff, 0, 0, 0);
-}
-__device__ __forceinline__ void lds_copy2(__amdgpu_buffer_rsrc_t r, uint8_t *lds, uint32_t voff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 2, voff, 0, 0, 0);
-}
-
 // this wavefront's copies into LDS complete, its LDS writes too, then the
 // workgroup barrier (no memory fence: the fence of __syncthreads would also
 // wait for the next stage's copies already in flight)
