@@ -473,15 +473,25 @@ int si_rope_kv_append(const si_shape_t *s, const float *qkv, int ldqkv, int ntok
     return check_launch("si_rope_kv_append");
 }
 
+// context splits, or what a causal prefill is sized by
 size_t si_attention_workspace(const si_shape_t *s, int nq, int max_ctx) {
     if (!s || nq <= 0 || max_ctx <= 0) return 0;
-    // context splits, or what a causal prefill is sized by
     const size_t a = attn_workspace_bytes(s->qheads, s->hdim, s->kvheads, nq, max_ctx);
     const size_t p = attn_prefill_workspace_bytes(s->qheads, s->hdim, nq);
     return a > p ? a : p;
 }
 
 }  // extern "C"
+
+// The least workspace a call takes: less than si_attention_workspace states
+// where the whole-row kernel has more chunks than the per-group one, which
+// runs then (the size such calls were documented with before).
+static size_t attention_least(const si_shape_t *s, int nq, int max_ctx) {
+    if (!s || nq <= 0 || max_ctx <= 0) return 0;
+    const size_t a = attn_workspace_min(s->qheads, s->hdim, s->kvheads, nq, max_ctx);
+    const size_t p = attn_prefill_workspace_bytes(s->qheads, s->hdim, nq);
+    return a > p ? a : p;
+}
 
 // Shared body of si_attention and si_attention_static: argument checks, then
 // the causal-prefill flash kernel or the split-context decode kernels with
@@ -504,8 +514,7 @@ static int attention_impl(const char *what, const si_shape_t *s, const float *q,
     }
     SI_REQUIRE(nq == 0 || (q && kc && vc && attn && ws), "%s: NULL pointer", what);
     SI_REQUIRE(!qs || d, "%s: qs without d", what);
-    SI_REQUIRE(ws_bytes >= si_attention_workspace(s, nq, max_ctx), "%s: workspace too small",
-               what);
+    SI_REQUIRE(ws_bytes >= attention_least(s, nq, max_ctx), "%s: workspace too small", what);
     if (!ctx_dev && ctx_step == 1 && kv_seq_stride == 0 && nq > 1 &&
         attn_prefill_supported(s->qheads, s->kvheads, s->hdim))
         // causal prefill of one sequence: the flash kernel (query i at
@@ -514,7 +523,7 @@ static int attention_impl(const char *what, const si_shape_t *s, const float *q,
                             bsum, S(stream));
     else
         launch_attention(q, nq, s->qheads, s->kvheads, s->hdim, kc, vc, kv_seq_stride, ctx_dev,
-                         ctx0, ctx_step, max_ctx, attn, qs, d, bsum, ws, S(stream));
+                         ctx0, ctx_step, max_ctx, attn, qs, d, bsum, ws, ws_bytes, S(stream));
     return check_launch(what);
 }
 
@@ -563,7 +572,7 @@ int si_attention_static(const si_shape_t *s, const float *q, int nq, const uint1
     int r = check_shape(s);
     if (r) return r;
     SI_REQUIRE(nq >= 0 && max_ctx >= 1, "si_attention_static: bad nq/max_ctx");
-    const size_t need = si_attention_workspace(s, nq, max_ctx);
+    const size_t need = attention_least(s, nq, max_ctx);
     SI_REQUIRE(need <= (size_t)SI_ATTENTION_STATIC_MAX,
                "si_attention_static: %d queries over max_ctx %d need %zu bytes of partial "
                "states, beyond the static buffer's %zu (use si_attention with a workspace)",
@@ -675,7 +684,7 @@ int si_attention_group(const si_shape_t *s, const float *q, int nheads, int grou
     const int kvd = s->kvheads * s->hdim;
     launch_attention(q, 1, nheads, 1, s->hdim, kc + (size_t)group * s->hdim,
                      vc + (size_t)group * s->hdim, 0, nullptr, context, 0, context, out, nullptr,
-                     nullptr, nullptr, ws, S(stream), KvPages(), kvd);
+                     nullptr, nullptr, ws, ws_bytes, S(stream), KvPages(), kvd);
     return check_launch("si_attention_group");
 }
 
@@ -1401,7 +1410,7 @@ static int run_rows(si_layer *L, const float *x, int rows, uint16_t *kc, uint16_
         else
             launch_attention(L->q, rows, s.qheads, s.kvheads, s.hdim, kc, vc, kv_seq_stride,
                              ctx_dev, ctx0, ctx_step, max_ctx, L->attn, L->attq.qs, L->attq.d,
-                             L->attq.s, L->attn_ws, st);
+                             L->attq.s, L->attn_ws, L->attn_ws_bytes, st);
     }
     mark(L, SI_PHASE_OUT_PROJ, st);
     if (!full) {
@@ -1569,7 +1578,7 @@ int si_attention_paged(const si_shape_t *s, const float *q, int nq, const uint16
     SI_REQUIRE(npages >= 1 && max_pages >= 1 && (long long)max_pages * page_size >= max_ctx,
                "attention_paged: pages do not cover max_ctx");
     SI_REQUIRE(!qs || d, "attention_paged: qs without d");
-    SI_REQUIRE(ws_bytes >= si_attention_workspace(s, nq, max_ctx),
+    SI_REQUIRE(ws_bytes >= attention_least(s, nq, max_ctx),
                "attention_paged: workspace too small");
     KvPages pg;
     pg.pages = pages;
@@ -1577,7 +1586,7 @@ int si_attention_paged(const si_shape_t *s, const float *q, int nq, const uint16
     pg.npages = npages;
     while ((1 << pg.shift) < page_size) ++pg.shift;
     launch_attention(q, nq, s->qheads, s->kvheads, s->hdim, k_pool, v_pool, 0, ctx_dev, max_ctx,
-                     0, max_ctx, attn, qs, d, bsum, ws, S(stream), pg);
+                     0, max_ctx, attn, qs, d, bsum, ws, ws_bytes, S(stream), pg);
     return check_launch("si_attention_paged");
 }
 

@@ -88,9 +88,11 @@ __global__ void k_attn_combine(int qheads, int hdim, int nsplit, const float *__
     float l = 0.0f, acc = 0.0f;
 #pragma unroll 8
     for (int s = 0; s < nsplit; ++s) {
-        const float w = expf(ws_m[base + s] - mx);  // empty chunk: m = -inf -> 0
+        // an empty chunk (m = -inf) weighs 0, and its output may be unwritten
+        const float ms = ws_m[base + s], w = __builtin_amdgcn_exp2f(ms - mx);
+        const float os = ws_o[(base + s) * hdim + jj];
         l = fmaf(ws_l[base + s], w, l);
-        acc = fmaf(ws_o[(base + s) * hdim + jj], w, acc);
+        acc = fmaf(ms == -INFINITY ? 0.0f : os, w, acc);
     }
     // context <= 0 (only possible through ctx_dev): zero output, as
     // attention_kernels.h:95-98 does
@@ -155,9 +157,11 @@ __global__ __launch_bounds__(1024) void k_attn_combine_wide(
     float l = 0.0f, acc = 0.0f;
 #pragma unroll 4
     for (int s = grp; s < nsplit; s += P) {
-        const float w = expf(ws_m[base + s] - mx);  // empty chunk: m = -inf -> 0
+        // an empty chunk (m = -inf) weighs 0, and its output may be unwritten
+        const float ms = ws_m[base + s], w = __builtin_amdgcn_exp2f(ms - mx);
+        const float os = ws_o[(base + s) * hdim + jj];
         l = fmaf(ws_l[base + s], w, l);
-        acc = fmaf(ws_o[(base + s) * hdim + jj], w, acc);
+        acc = fmaf(ms == -INFINITY ? 0.0f : os, w, acc);
     }
     red_o[tid] = acc;
     if (jj == 0) red_l[grp] = l;
@@ -241,7 +245,7 @@ template <int D>
 __global__ void __launch_bounds__(256) k_attn_decode_mfma(
     const float *__restrict__ q, int qheads, int kvheads, const uint16_t *__restrict__ kc,
     const uint16_t *__restrict__ vc, size_t kv_seq_stride, const int *__restrict__ ctx_dev,
-    int ctx0, int ctx_step, int max_ctx, int chunk, float scale, float *__restrict__ ws_m,
+    int ctx0, int ctx_step, int max_ctx, int chunk, float scale2, float *__restrict__ ws_m,
     float *__restrict__ ws_l, float *__restrict__ ws_o, KvPages pg, int kv_row) {
     constexpr int KS = D / 32;  // k-steps of the score MFMA
     constexpr int DT = D / 16;  // d-tiles of the PV MFMA
@@ -300,30 +304,33 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
             const int kpos = min(t0 + col, p1 - 1);
             const uint16_t *krow = kbase + pg.row(qi, kpos, kv_seq_stride, kvd) + 8 * grp;
             f4 sacc = (f4){0.f, 0.f, 0.f, 0.f};
+            h8 ka[KS];
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const uint4 kraw = *(const uint4 *)(krow + 32 * ks);
-                const h8 ka = __builtin_bit_cast(h8, kraw);
-                sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qh[ks], sacc, 0, 0, 0);
-                sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[ks], sacc, 0, 0, 0);
-            }
+            for (int ks = 0; ks < KS; ++ks) ka[ks] = *(const h8 *)(krow + 32 * ks);
+            // the lo products first: they round at their own small magnitude
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], ql[ks], sacc, 0, 0, 0);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], qh[ks], sacc, 0, 0, 0);
             // lane holds S^T[pos = t0 + 4*grp + r][head = col]
             float s[4];
             float mx = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int pos = t0 + 4 * grp + r;
-                s[r] = pos < p1 ? sacc[r] * scale : -INFINITY;
+                s[r] = pos < p1 ? sacc[r] : -INFINITY;
                 mx = fmaxf(mx, s[r]);
             }
             mx = fmaxf(mx, swap16_f(mx));
             mx = fmaxf(mx, swap32_f(mx));
-            const float mnew = fmaxf(m, mx);
-            const float alpha = expf(m - mnew);  // 0 while m is -inf
+            const float mnew = fmaxf(m, mx * scale2);
+            const float alpha = __builtin_amdgcn_exp2f(m - mnew);  // 0 while m is -inf
             float p[4], ps = 0.0f;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                p[r] = expf(s[r] - mnew);
+                p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], scale2, -mnew));
                 ps += p[r];
             }
             ps += swap16_f(ps);
@@ -364,7 +371,7 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
     }
     __syncthreads();
     const float mall = fmaxf(fmaxf(mrg_m[0][col], mrg_m[1][col]), fmaxf(mrg_m[2][col], mrg_m[3][col]));
-    const float w = m == -INFINITY ? 0.0f : expf(m - mall);  // a wave with no positions adds 0
+    const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mall);  // a wave with no positions adds 0
     for (int k = 0; k < 4; ++k) {
         if (wave == k)
 #pragma unroll
@@ -381,7 +388,7 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
     if (wave == 0 && grp == 0 && col < per) {
         float l = 0.0f;
         for (int k = 0; k < 4; ++k)
-            if (mrg_m[k][col] != -INFINITY) l += mrg_l[k][col] * expf(mrg_m[k][col] - mall);
+            if (mrg_m[k][col] != -INFINITY) l += mrg_l[k][col] * __builtin_amdgcn_exp2f(mrg_m[k][col] - mall);
         ws_m[pbase + (size_t)col * nsplit] = mall;
         ws_l[pbase + (size_t)col * nsplit] = l;
     }
@@ -815,8 +822,7 @@ void launch_attn_prefill(const float *q, int ntok, int qheads, int kvheads, int 
                          uint16_t *qd, int16_t *bsum, hipStream_t st) {
     if (ntok <= 0) return;
     const int per = qheads / kvheads;
-    // scores in powers of two: exp(s / sqrt(hdim)) (attention_kernels.h:86)
-    const float scale2 = 1.44269504088896340736f / sqrtf((float)hdim);
+    const float scale2 = softmax_scale2(hdim);
     // Wavefronts per workgroup, by the number of 32-row tiles.  While they are
     // fewer than two per CU each tile gets a workgroup of its own, its range
     // walked four ways; past that two or four tiles share each staged K/V
@@ -872,8 +878,33 @@ int attn_nsplit(int kvheads, int nq, int max_ctx) {
     return ns < 1 ? 1 : ns;
 }
 
-size_t attn_workspace_bytes(int qheads, int hdim, int kvheads, int nq, int max_ctx) {
+size_t attn_workspace_min(int qheads, int hdim, int kvheads, int nq, int max_ctx) {
     const int ns = attn_nsplit(kvheads, nq, max_ctx);  // one partial per workgroup
+    return (size_t)nq * qheads * ns * (hdim + 2) * sizeof(float);
+}
+
+// Context chunks of the whole-row kernel for si_attention's queries (0: not
+// its shape, the per-group kernel runs): at least four steps each, about 512
+// workgroups in all (two per CU; workgroups past a query's context leave at
+// once), no more than 31 (32 take the wide merge: 4.4 -> 8-10 us), and
+// partials within 16 MB or the per-group kernel's.  Measured (us, kernel +
+// merge; per-group kernel -> this, 512 | 1024 workgroups aimed at): 48 queries
+// x 200-4096 positions (7B heads) 104.7 + 4.1 -> 51.5 + 4.5 | 50.9 + 6.9; 64 x
+// 4096 157 + 4.2 -> 94.8 + 4.2 | 98.3 + 4.5; 20 x 1000-4000 43.7 + 4.4 -> 19.9 +
+// 4.4 | 24 + 9; 0.5B heads, 64 x 10-4000 35.5 + 4.1 -> 18.2 + 4.1, 24 x 100-2048
+// 11.8 + 4.0 -> 7.6 + 4.0; 8 x 1-300 (7B) 9.4 + 4.0 -> 7.4 + 4.0.
+static int attn_rows_nsplit(int qheads, int kvheads, int hdim, int nq, int max_ctx) {
+    if (!dec_rows_ok(qheads, kvheads, hdim, nq)) return 0;
+    const int rows = 16 * (4 / kvheads);
+    const int ns = min((max_ctx + 4 * rows - 1) / (4 * rows), (512 + nq - 1) / nq);
+    const size_t each = (size_t)nq * qheads * (hdim + 2) * sizeof(float);
+    const int most = max((int)(((size_t)16 << 20) / each), attn_nsplit(kvheads, nq, max_ctx));
+    return max(1, min(ns, min(most, 31)));
+}
+
+size_t attn_workspace_bytes(int qheads, int hdim, int kvheads, int nq, int max_ctx) {
+    const int ns = max(attn_nsplit(kvheads, nq, max_ctx),
+                       attn_rows_nsplit(qheads, kvheads, hdim, nq, max_ctx));
     return (size_t)nq * qheads * ns * (hdim + 2) * sizeof(float);
 }
 
@@ -885,21 +916,30 @@ bool attn_supported(int qheads, int kvheads, int hdim) {
 void launch_attention(const float *q, int nq, int qheads, int kvheads, int hdim,
                       const uint16_t *kc, const uint16_t *vc, size_t kv_seq_stride,
                       const int *ctx_dev, int ctx0, int ctx_step, int max_ctx, float *attn,
-                      int8_t *qs, uint16_t *d, int16_t *bsum, void *workspace,
+                      int8_t *qs, uint16_t *d, int16_t *bsum, void *workspace, size_t ws_bytes,
                       hipStream_t st, KvPages pg, int kv_row) {
     if (nq <= 0) return;
     if (kv_row <= 0) kv_row = kvheads * hdim;
+    const int nr = attn_rows_nsplit(qheads, kvheads, hdim, nq, max_ctx);
+    if (nr > 0 && kv_row == kvheads * hdim &&
+        ws_bytes >= (size_t)nq * qheads * nr * (hdim + 2) * sizeof(float) &&
+        (((uintptr_t)q | (uintptr_t)workspace) & 15) == 0) {
+        launch_attn_rows(q, nq, qheads, kvheads, hdim, kc, vc, kv_seq_stride, ctx_dev, ctx0,
+                         ctx_step, max_ctx, nr, workspace, st, pg);
+        launch_attn_combine(nq, qheads, hdim, nr, workspace, attn, qs, d, bsum, st);
+        return;
+    }
     const int ns = attn_nsplit(kvheads, nq, max_ctx);
     int chunk = (max_ctx + ns - 1) / ns;
     chunk = (chunk + MA_SUPER - 1) / MA_SUPER * MA_SUPER;
     float *ws_m = (float *)workspace;
     float *ws_l = ws_m + (size_t)nq * qheads * ns;
     float *ws_o = ws_l + (size_t)nq * qheads * ns;
-    const float scale = 1.0f / sqrtf((float)hdim);  // attention_kernels.h:86
+    const float scale2 = softmax_scale2(hdim);
     const dim3 grid(ns, kvheads, nq);
 #define SI_ATTN_LAUNCH(DIM)                                                                  \
     SI_LAUNCH(k_attn_decode_mfma<DIM>, grid, dim3(256), 0, st, q, qheads, kvheads, kc,       \
-              vc, kv_seq_stride, ctx_dev, ctx0, ctx_step, max_ctx, chunk, scale, ws_m,       \
+              vc, kv_seq_stride, ctx_dev, ctx0, ctx_step, max_ctx, chunk, scale2, ws_m,      \
               ws_l, ws_o, pg, kv_row)
     switch (hdim) {
         case 32: SI_ATTN_LAUNCH(32); break;

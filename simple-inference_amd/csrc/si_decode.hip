@@ -199,8 +199,9 @@ __global__ void __launch_bounds__(T) k_dec_qkv(
 // ---------------------------------------------------------------------------
 // 3: merge attention partials -> attn fp32 -> Q8 -> W_O mat-vec (+ residual)
 // ---------------------------------------------------------------------------
-// Partials per (head, chunk s): running max m, sum l, unnormalised o[D].
-// attn[h][d] = sum_s o_s[d] e^(m_s - M) * (1 / sum_s l_s e^(m_s - M)),
+// Partials per (head, chunk s): running max m (in powers of two), sum l,
+// unnormalised o[D].
+// attn[h][d] = sum_s o_s[d] 2^(m_s - M) * (1 / sum_s l_s 2^(m_s - M)),
 // M = max_s m_s; a head with no context (M = -inf) gives 0
 // (attention_kernels.h:95-98).
 template <int R, int T, bool EXACT>
@@ -223,7 +224,7 @@ __global__ void __launch_bounds__(T) k_dec_wo(
                                          RowIdentity{});
     // Thread t merges the 4 consecutive elements 4*e4.. (e4 = t + T*i), 8
     // chunks at a time, with the online rule (m, l, o) <- (M',
-    // l e^(m-M') + l_s e^(m_s-M'), o e^(m-M') + o_s e^(m_s-M')), then
+    // l 2^(m-M') + l_s 2^(m_s-M'), o 2^(m-M') + o_s 2^(m_s-M')), then
     // quantizes: 8 consecutive lanes hold one Q8_0 block of the output
     // (qwen_one_layer.c:272).  The first group of partials is requested
     // before the weights, which then load while the merge runs.  A
@@ -260,9 +261,8 @@ __global__ void __launch_bounds__(T) k_dec_wo(
             for (int u = 0; u < SC; ++u) {
                 if (s0 + u >= ns || om[u] == -INFINITY) continue;  // empty chunk
                 const float mn = fmaxf(M, om[u]);
-                // hardware exp2, as in the attention's own online softmax
-                const float a = M == -INFINITY ? 0.0f : __expf(M - mn);
-                const float bw = __expf(om[u] - mn);
+                const float a = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - mn);
+                const float bw = __builtin_amdgcn_exp2f(om[u] - mn);
                 A[0] = fmaf(oo[u].x, bw, A[0] * a);
                 A[1] = fmaf(oo[u].y, bw, A[1] * a);
                 A[2] = fmaf(oo[u].z, bw, A[2] * a);
@@ -421,7 +421,7 @@ __global__ void __launch_bounds__(NW * 64) k_dec_attn(
     const float *__restrict__ qkv, int ldqkv, int qheads, int kvheads,
     const float *__restrict__ rc, const float *__restrict__ rs, uint16_t *__restrict__ kc,
     uint16_t *__restrict__ vc, size_t kv_seq_stride, const int *__restrict__ ctx_dev, int ctx0,
-    int max_ctx, int chunk, float scale, float *__restrict__ q_cap, float *__restrict__ ws_m,
+    int max_ctx, int chunk, float scale2, float *__restrict__ q_cap, float *__restrict__ ws_m,
     float *__restrict__ ws_l, float *__restrict__ ws_o, float *__restrict__ attn,
     int8_t *__restrict__ aqs, uint16_t *__restrict__ ad, int16_t *__restrict__ as, KvPages pg,
     DecQkvIn fq) {
@@ -676,28 +676,31 @@ __global__ void __launch_bounds__(NW * 64) k_dec_attn(
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) ka[ks] = __builtin_bit_cast(h8, kr[ks]);
         f4 sacc = (f4){0.f, 0.f, 0.f, 0.f};
+        // the lo products first: they round at their own small magnitude
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], qh[ks], sacc, 0, 0, 0);
+        for (int ks = 0; ks < KS; ++ks)
             sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], ql[ks], sacc, 0, 0, 0);
-        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], qh[ks], sacc, 0, 0, 0);
         // lane holds S^T[pos = t0 + 4*grp + r][head col]
         float s[4], mx = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            s[r] = (t0 + 4 * grp + r < p1) ? sacc[r] * scale : -INFINITY;
+            s[r] = (t0 + 4 * grp + r < p1) ? sacc[r] : -INFINITY;
             mx = fmaxf(mx, s[r]);
         }
         mx = fmaxf(mx, swap16_f(mx));
         mx = fmaxf(mx, swap32_f(mx));
-        const float mnew = fmaxf(m, mx);
-        // hardware exp2 (relative error ~1e-6 here, far inside the 2e-3
-        // attention tolerance); mnew is finite from the first tile on
-        const float alpha = __expf(m - mnew);  // 0 while m is -inf
+        // m and the weights in powers of two (scale2 = log2(e) / sqrt(D)): one
+        // fma and the hardware exponential per score; mnew is finite from the
+        // first tile on
+        const float mnew = fmaxf(m, mx * scale2);
+        const float alpha = __builtin_amdgcn_exp2f(m - mnew);  // 0 while m is -inf
         float p[4], ps = 0.0f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            p[r] = __expf(s[r] - mnew);
+            p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], scale2, -mnew));
             ps += p[r];
         }
         ps += swap16_f(ps);
@@ -776,7 +779,7 @@ __global__ void __launch_bounds__(NW * 64) k_dec_attn(
     __syncthreads();
     // 4 consecutive elements per thread; 8 lanes = 32 elements = one Q8_0
     // block of one head (D is a multiple of 32).  Each thread forms its
-    // head's M = max over wavefronts, the factors e^(m_w - M) and the total
+    // head's M = max over wavefronts, the factors 2^(m_w - M) and the total
     // l itself (broadcast LDS reads; no further barrier).
     const int nel4 = nh * D / 4;
     for (int e40 = 0; e40 < nel4; e40 += NW * 64) {
@@ -791,8 +794,8 @@ __global__ void __launch_bounds__(NW * 64) k_dec_attn(
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
             const float4 ov = *(const float4 *)(mo + ((size_t)w * nh + hc) * D + dd);
-            // hardware exp2, as in the tile loop; an empty wavefront gives 0
-            const float f = M == -INFINITY ? 0.0f : __expf(mm[w * nh + hc] - M);
+            // an empty wavefront gives 0
+            const float f = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mm[w * nh + hc] - M);
             ltot = fmaf(ml[w * nh + hc], f, ltot);
             acc[0] = fmaf(ov.x, f, acc[0]);
             acc[1] = fmaf(ov.y, f, acc[1]);
@@ -864,14 +867,16 @@ struct RowsLds {
     }
 };
 
-template <int D, int G, bool FINAL, bool PAGED>
+// RAW (si_attention): qkv holds rotated queries only ([nq][qheads * D]) and
+// every position's row is in the cache: no rotation, nothing appended.
+template <int D, int G, bool FINAL, bool PAGED, bool RAW>
 __global__ void __launch_bounds__(256) k_dec_attn_rows(
     const float *__restrict__ qkv, int ldqkv, int qheads, const float *__restrict__ rc,
     const float *__restrict__ rs, uint16_t *__restrict__ kc, uint16_t *__restrict__ vc,
     size_t kv_seq_stride, const int *__restrict__ ctx_dev, int ctx0, int max_ctx, int chunk,
-    float scale, float *__restrict__ q_cap, float *__restrict__ ws_m, float *__restrict__ ws_l,
+    float scale2, float *__restrict__ q_cap, float *__restrict__ ws_m, float *__restrict__ ws_l,
     float *__restrict__ ws_o, float *__restrict__ attn, int8_t *__restrict__ aqs,
-    uint16_t *__restrict__ ad, int16_t *__restrict__ as, KvPages pg) {
+    uint16_t *__restrict__ ad, int16_t *__restrict__ as, KvPages pg, int ctx_step) {
     using L = RowsLds<D, G>;
     constexpr int KS = D / 32, DT = D / 16, HALF = D / 2, NWG = L::NWG, ROWS = L::ROWS;
     constexpr int RW = L::RW, KVD = G * D;
@@ -896,15 +901,28 @@ __global__ void __launch_bounds__(256) k_dec_attn_rows(
     const int g = wave % G, wj = wave / G;  // group, tile slot within the step
     const int per = qheads / G;
     const int qd = qheads * D;
-    int ctx = ctx_dev ? ctx_dev[qi] : ctx0;
+    int ctx = ctx_dev ? ctx_dev[qi] : ctx0 + qi * ctx_step;
     ctx = min(ctx, max_ctx);
     const int pnew = ctx - 1;  // < 0: empty context (device-supplied only)
     const int p0 = sp * chunk;
     const int p1 = min(ctx, p0 + chunk);
     // rows the loads may touch: known at launch, so the first loads need not
-    // wait for ctx_dev (the cache holds max_ctx rows per sequence)
-    const int pmax = min(max_ctx, p0 + chunk);
-    const bool owner = pnew >= p0 && pnew < p1;
+    // wait for ctx_dev (a layer's cache holds max_ctx rows per sequence;
+    // si_attention's callers owe only the rows of each context)
+    const int pmax = RAW ? p1 : min(max_ctx, p0 + chunk);
+    const bool owner = !RAW && pnew >= p0 && pnew < p1;
+    if constexpr (RAW && !FINAL) {
+        // a chunk past the query's context leaves an empty state (ragged
+        // contexts: such workgroups are the rule, and cost no row loads)
+        if (p0 >= p1) {
+            for (int h = tid; h < qheads; h += 256) {
+                const size_t pi = ((size_t)qi * qheads + h) * ns + sp;
+                ws_m[pi] = -INFINITY;
+                ws_l[pi] = 0.0f;
+            }
+            return;
+        }
+    }
     const float *row = qkv + (size_t)qi * ldqkv;
     const float *cr = rc + (size_t)max(pnew, 0) * HALF;
     const float *sr = rs + (size_t)max(pnew, 0) * HALF;
@@ -917,14 +935,14 @@ __global__ void __launch_bounds__(256) k_dec_attn_rows(
     float *kraw = qraw + G * per * D;  // [G][D]
     float *vraw = kraw + KVD;          // [G][D]
     float *csr = vraw + KVD;           // [HALF] cos, [HALF] sin
-    const int nrow4 = (qd + 2 * KVD) / 4;
+    const int nrow4 = (RAW ? qd : qd + 2 * KVD) / 4;
     constexpr int ROW4PT = ((16 + 2) * G * D / 4 + 255) / 256;  // per <= 16
     float4 rv[ROW4PT];
 #pragma unroll
     for (int u = 0; u < ROW4PT; ++u)
         rv[u] = ((const float4 *)row)[min(tid + u * 256, nrow4 - 1)];
-    float4 csv;
-    {
+    float4 csv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if constexpr (!RAW) {
         const int t = min(tid, D / 4 - 1);
         const float4 *cp = t < HALF / 4 ? (const float4 *)cr + t : (const float4 *)sr + (t - HALF / 4);
         csv = *cp;
@@ -953,7 +971,7 @@ __global__ void __launch_bounds__(256) k_dec_attn_rows(
     // K/V loads above and wait for all of them
 #pragma unroll
     for (int u = 0; u < ROW4PT; ++u) ((float4 *)qraw)[min(tid + u * 256, nrow4 - 1)] = rv[u];
-    ((float4 *)csr)[min(tid, D / 4 - 1)] = csv;
+    if constexpr (!RAW) ((float4 *)csr)[min(tid, D / 4 - 1)] = csv;
     __syncthreads();
     // rotate-half RoPE (qwen_one_layer.c:172-183) of element dd of a head row
     auto rot = [&](const float *v, int dd) {
@@ -965,6 +983,7 @@ __global__ void __launch_bounds__(256) k_dec_attn_rows(
     // the new token's K (rotated) and V rows in fp16, for every group (a
     // constant trip count: a loop with stores and no loads makes the
     // compiler drain every load in flight before it)
+    if constexpr (!RAW)
 #pragma unroll
     for (int u = 0; u < (KVD + 255) / 256; ++u) {
         const int i = tid + 256 * u;
@@ -996,15 +1015,23 @@ __global__ void __launch_bounds__(256) k_dec_attn_rows(
             const int d0 = 32 * ks + 8 * grp;
             const int i0 = d0 < HALF ? d0 : d0 - HALF;
             float a[8], b[8], c[8], sn[8], v[8];
-            ld8(qh_row + i0, a);
-            ld8(qh_row + i0 + HALF, b);
-            ld8(csr + i0, c);
-            ld8(csr + HALF + i0, sn);
+            if constexpr (RAW) {
+                ld8(qh_row + d0, a);
+            } else {
+                ld8(qh_row + i0, a);
+                ld8(qh_row + i0 + HALF, b);
+                ld8(csr + i0, c);
+                ld8(csr + HALF + i0, sn);
+            }
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                v[e] = !hv ? 0.0f
-                           : (d0 < HALF ? __fsub_rn(__fmul_rn(a[e], c[e]), __fmul_rn(b[e], sn[e]))
-                                        : __fadd_rn(__fmul_rn(b[e], c[e]), __fmul_rn(a[e], sn[e])));
+                if constexpr (RAW)
+                    v[e] = hv ? a[e] : 0.0f;
+                else
+                    v[e] = !hv ? 0.0f
+                               : (d0 < HALF
+                                      ? __fsub_rn(__fmul_rn(a[e], c[e]), __fmul_rn(b[e], sn[e]))
+                                      : __fadd_rn(__fmul_rn(b[e], c[e]), __fmul_rn(a[e], sn[e])));
                 _Float16 hi, lo;
                 hi_lo(v[e], hi, lo);
                 qh[ks][e] = hi;
@@ -1065,28 +1092,30 @@ __global__ void __launch_bounds__(256) k_dec_attn_rows(
         for (int ks = 0; ks < KS; ++ks)
             ka[ks] = *(const h8 *)(kt + (DA_TILE * wj + col) * RW + g * D + 32 * ks + 8 * grp);
         f4 sacc = (f4){0.f, 0.f, 0.f, 0.f};
+        // the lo products first: they round at their own small magnitude
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], qh[ks], sacc, 0, 0, 0);
+        for (int ks = 0; ks < KS; ++ks)
             sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], ql[ks], sacc, 0, 0, 0);
-        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], qh[ks], sacc, 0, 0, 0);
         // lane holds S^T[pos = t0 + 4*grp + r][head col]
         float s[4], mx = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            s[r] = (t0 + 4 * grp + r < p1) ? sacc[r] * scale : -INFINITY;
+            s[r] = (t0 + 4 * grp + r < p1) ? sacc[r] : -INFINITY;
             mx = fmaxf(mx, s[r]);
         }
         mx = fmaxf(mx, swap16_f(mx));
         mx = fmaxf(mx, swap32_f(mx));
-        const float mnew = fmaxf(m, mx);
+        const float mnew = fmaxf(m, mx * scale2);  // in powers of two, as k_dec_attn's
         // a tile past the chunk end leaves the state as it is (no NaN)
         const float mref = mnew == -INFINITY ? 0.0f : mnew;
-        const float alpha = __expf(m - mref);
+        const float alpha = __builtin_amdgcn_exp2f(m - mref);
         float p[4], ps_ = 0.0f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            p[r] = __expf(s[r] - mref);
+            p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], scale2, -mref));
             ps_ += p[r];
         }
         ps_ += swap16_f(ps_);
@@ -1174,7 +1203,8 @@ __global__ void __launch_bounds__(256) k_dec_attn_rows(
         float l = 0.0f;
 #pragma unroll
         for (int w = 0; w < NWG; ++w) {
-            const float f = M == -INFINITY ? 0.0f : expf(mm[(gg * NWG + w) * per + hc] - M);
+            const float f =
+                M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mm[(gg * NWG + w) * per + hc] - M);
             sc[tid * NWG + w] = f;
             l = fmaf(ml[(gg * NWG + w) * per + hc], f, l);
         }
@@ -1304,7 +1334,7 @@ constexpr size_t ROWS_LDS_MAX = 80 * 1024;
 // The whole-row kernel serves batches (>= 8 queries: one query is latency
 // bound and k_dec_attn's shorter chain wins) of 1, 2 or 4 KV groups of up to
 // 16 query heads.
-static bool dec_rows_ok(int qheads, int kvheads, int hdim, int nq) {
+bool dec_rows_ok(int qheads, int kvheads, int hdim, int nq) {
     if (nq < 8 || !(kvheads == 1 || kvheads == 2 || kvheads == 4)) return false;
     if (qheads % kvheads || qheads / kvheads > 16) return false;
     const int per = qheads / kvheads;
@@ -1380,7 +1410,7 @@ static void dec_attn_impl(const float *qkv, int ldqkv, int nq, int qheads, int k
     float *ws_m = (float *)workspace;
     float *ws_l = ws_m + (size_t)nq * qheads * ns;
     float *ws_o = ws_l + (size_t)nq * qheads * ns;
-    const float scale = 1.0f / sqrtf((float)hdim);  // attention_kernels.h:86
+    const float scale2 = softmax_scale2(hdim);
     const int per = qheads / kvheads;
     const bool fin = attn != nullptr;
     if (dec_rows_ok(qheads, kvheads, hdim, nq)) {
@@ -1389,15 +1419,15 @@ static void dec_attn_impl(const float *qkv, int ldqkv, int nq, int qheads, int k
         static bool big_lds = false;                                                              \
         if (!big_lds) {                                                                           \
             /* past 64 KB of dynamic LDS; a failure surfaces as the launch's error */            \
-            (void)hipFuncSetAttribute((const void *)k_dec_attn_rows<DIM, GG, FIN, PAGED>,         \
+            (void)hipFuncSetAttribute((const void *)k_dec_attn_rows<DIM, GG, FIN, PAGED, false>,  \
                                       hipFuncAttributeMaxDynamicSharedMemorySize,                 \
                                       (int)ROWS_LDS_MAX);                                         \
             big_lds = true;                                                                       \
         }                                                                                         \
-        SI_LAUNCH((k_dec_attn_rows<DIM, GG, FIN, PAGED>), dim3(ns, nq), dim3(256),                \
+        SI_LAUNCH((k_dec_attn_rows<DIM, GG, FIN, PAGED, false>), dim3(ns, nq), dim3(256),         \
                   (RowsLds<DIM, GG>::bytes(per)), st, qkv, ldqkv, qheads, rc, rs, kc, vc,         \
-                  kv_seq_stride, ctx_dev, ctx0, max_ctx, chunk, scale, q_cap, ws_m, ws_l,         \
-                  ws_o, attn, aqs, ad, as, pg);                                                   \
+                  kv_seq_stride, ctx_dev, ctx0, max_ctx, chunk, scale2, q_cap, ws_m, ws_l,         \
+                  ws_o, attn, aqs, ad, as, pg, 0);                                                \
     } while (0)
 #define RCALLG(DIM)                                                \
     if (kvheads == 1) {                                            \
@@ -1421,7 +1451,7 @@ static void dec_attn_impl(const float *qkv, int ldqkv, int nq, int qheads, int k
 #define CALL(DIM, NW, FIN, DEP)                                                                \
     SI_LAUNCH((k_dec_attn<DIM, NW, FIN, PAGED, DEP>), grid, dim3(NW * 64),                     \
               (AttnLds<DIM, NW>::bytes(per)), st, qkv, ldqkv, qheads, kvheads, rc, rs,         \
-              kc, vc, kv_seq_stride, ctx_dev, ctx0, max_ctx, chunk, scale, q_cap,              \
+              kc, vc, kv_seq_stride, ctx_dev, ctx0, max_ctx, chunk, scale2, q_cap,              \
               ws_m, ws_l, ws_o, attn, aqs, ad, as, pg, DecQkvIn{})
 #define CALLN(DIM, NW, FIN)                                             \
     if (chunk <= DA_TILE * NW) {                                        \
@@ -1457,6 +1487,61 @@ static void dec_attn_impl(const float *qkv, int ldqkv, int nq, int qheads, int k
 #undef CALL
 }
 
+// Whole-row attention of si_attention's queries (RAW): partials [nq][qheads]
+// [ns] as k_dec_attn's, for launch_attn_combine.
+template <bool PAGED>
+static void attn_rows_impl(const float *q, int nq, int qheads, int kvheads, int hdim,
+                           const uint16_t *kc, const uint16_t *vc, size_t kv_seq_stride,
+                           const int *ctx_dev, int ctx0, int ctx_step, int max_ctx, int ns,
+                           void *workspace, hipStream_t st, KvPages pg) {
+    const int chunk = ((max_ctx + ns - 1) / ns + DA_TILE - 1) / DA_TILE * DA_TILE;
+    float *ws_m = (float *)workspace;
+    float *ws_l = ws_m + (size_t)nq * qheads * ns;
+    float *ws_o = ws_l + (size_t)nq * qheads * ns;
+    const float scale2 = softmax_scale2(hdim);
+    const int per = qheads / kvheads;
+#define RCALL(DIM, GG)                                                                           \
+    do {                                                                                         \
+        static bool big_lds = false;                                                             \
+        if (!big_lds) {                                                                          \
+            /* past 64 KB of dynamic LDS; a failure surfaces as the launch's error */           \
+            (void)hipFuncSetAttribute((const void *)k_dec_attn_rows<DIM, GG, false, PAGED, true>, \
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,                \
+                                      (int)ROWS_LDS_MAX);                                        \
+            big_lds = true;                                                                      \
+        }                                                                                        \
+        SI_LAUNCH((k_dec_attn_rows<DIM, GG, false, PAGED, true>), dim3(ns, nq), dim3(256),       \
+                  (RowsLds<DIM, GG>::bytes(per)), st, q, qheads *hdim, qheads, nullptr, nullptr, \
+                  const_cast<uint16_t *>(kc), const_cast<uint16_t *>(vc), kv_seq_stride,         \
+                  ctx_dev, ctx0, max_ctx, chunk, scale2, nullptr, ws_m, ws_l, ws_o, nullptr,      \
+                  nullptr, nullptr, nullptr, pg, ctx_step);                                      \
+    } while (0)
+#define RCALLG(DIM)                      \
+    if (kvheads == 1) RCALL(DIM, 1);     \
+    else if (kvheads == 2) RCALL(DIM, 2); \
+    else RCALL(DIM, 4)
+    switch (hdim) {
+        case 32: RCALLG(32); break;
+        case 64: RCALLG(64); break;
+        case 96: RCALLG(96); break;
+        default: RCALLG(128); break;
+    }
+#undef RCALLG
+#undef RCALL
+}
+
+void launch_attn_rows(const float *q, int nq, int qheads, int kvheads, int hdim,
+                      const uint16_t *kc, const uint16_t *vc, size_t kv_seq_stride,
+                      const int *ctx_dev, int ctx0, int ctx_step, int max_ctx, int ns,
+                      void *workspace, hipStream_t st, KvPages pg) {
+    if (pg.pages)
+        attn_rows_impl<true>(q, nq, qheads, kvheads, hdim, kc, vc, kv_seq_stride, ctx_dev, ctx0,
+                             ctx_step, max_ctx, ns, workspace, st, pg);
+    else
+        attn_rows_impl<false>(q, nq, qheads, kvheads, hdim, kc, vc, kv_seq_stride, ctx_dev, ctx0,
+                              ctx_step, max_ctx, ns, workspace, st, pg);
+}
+
 // Single-token decode with the Q|K|V projection inside the attention
 // (k_dec_attn<..., FQ>): worth it while a workgroup's 3*hdim weight rows
 // stream in well under a kernel boundary (0.5B: 97 KB); 7B's 384 rows of
@@ -1480,14 +1565,14 @@ void launch_dec_qkv_attn(const DecQkvIn &fq, int qheads, int kvheads, int hdim, 
     float *ws_m = (float *)workspace;
     float *ws_l = ws_m + (size_t)qheads * ns;
     float *ws_o = ws_l + (size_t)qheads * ns;
-    const float scale = 1.0f / sqrtf((float)hdim);  // attention_kernels.h:86
+    const float scale2 = softmax_scale2(hdim);
     const dim3 grid(ns, qheads, 1);
 #define FQCALL(DIM, DEP)                                                                       \
     SI_LAUNCH((k_dec_attn<DIM, DA_NW, false, false, DEP, true>), grid, dim3(DA_NW * 64),       \
               ((AttnLds<DIM, DA_NW>::bytes(1) + 15) / 16 * 16 +                                \
                FqLds<DIM, DA_NW>::bytes(fq.hidden)),                                           \
               st, nullptr, 0, qheads, kvheads, rc, rs, kc, vc, (size_t)0, nullptr, ctx, ctx,   \
-              chunk, scale, q_cap, ws_m, ws_l, ws_o, nullptr, nullptr, nullptr, nullptr,       \
+              chunk, scale2, q_cap, ws_m, ws_l, ws_o, nullptr, nullptr, nullptr, nullptr,       \
               KvPages(), fq)
     const bool one = chunk <= DA_TILE * DA_NW;
     if (hdim == 64) {

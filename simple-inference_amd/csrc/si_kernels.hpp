@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stddef.h>
 #include <atomic>
 #include <stdint.h>
@@ -177,8 +178,15 @@ void launch_rope_kv(const float *qkv, int ldqkv, int ntok, int qheads, int kvhea
                     int pos0, int pos_step, int max_pos, const int *ctx_dev, const float *rc,
                     const float *rs, float *q_out, uint16_t *kc, uint16_t *vc,
                     size_t kv_seq_stride, hipStream_t st, KvPages pg = KvPages());
+// The attention kernels' softmax runs in powers of two: exp(s / sqrt(hdim))
+// (attention_kernels.h:86) = 2^(s * softmax_scale2), and the running maxima of
+// every partial state (ws_m) are in that scale.
+inline float softmax_scale2(int hdim) { return 1.44269504088896340736f / sqrtf((float)hdim); }
 int attn_nsplit(int kvheads, int nq, int max_ctx);
+// Partial states of launch_attention: what it runs best with, and the least
+// it takes (fewer, longer context chunks).
 size_t attn_workspace_bytes(int qheads, int hdim, int kvheads, int nq, int max_ctx);
+size_t attn_workspace_min(int qheads, int hdim, int kvheads, int nq, int max_ctx);
 bool attn_supported(int qheads, int kvheads, int hdim);
 // three-stage textbook attention for one query (scores: [qheads][ctx] fp32)
 bool attn_standard_supported(int qheads, int kvheads, int hdim);
@@ -187,7 +195,7 @@ void launch_attn_standard(const float *q, int qheads, int kvheads, int hdim, con
 void launch_attention(const float *q, int nq, int qheads, int kvheads, int hdim,
                       const uint16_t *kc, const uint16_t *vc, size_t kv_seq_stride,
                       const int *ctx_dev, int ctx0, int ctx_step, int max_ctx, float *attn,
-                      int8_t *qs, uint16_t *d, int16_t *bsum, void *workspace,
+                      int8_t *qs, uint16_t *d, int16_t *bsum, void *workspace, size_t ws_bytes,
                       hipStream_t st, KvPages pg = KvPages(), int kv_row = 0);
 bool attn_prefill_supported(int qheads, int kvheads, int hdim);
 size_t attn_prefill_workspace_bytes(int qheads, int hdim, int ntok);
@@ -211,6 +219,14 @@ void launch_dec_gateup(const float *h, const float *gain, int hidden, float eps,
                        int8_t *cap_qs, uint16_t *cap_d, int16_t *cap_s, float *gu, float *act,
                        int8_t *aqs, uint16_t *ad, int16_t *as, bool exact, hipStream_t st);
 int dec_attn_chunks(int qheads, int kvheads, int hdim, int nq, int max_ctx);
+// Whether the whole-row attention kernel takes a batch of nq queries, and that
+// kernel over si_attention's queries (partials [nq][qheads][ns] for
+// launch_attn_combine).
+bool dec_rows_ok(int qheads, int kvheads, int hdim, int nq);
+void launch_attn_rows(const float *q, int nq, int qheads, int kvheads, int hdim,
+                      const uint16_t *kc, const uint16_t *vc, size_t kv_seq_stride,
+                      const int *ctx_dev, int ctx0, int ctx_step, int max_ctx, int ns,
+                      void *workspace, hipStream_t st, KvPages pg);
 // The layer input, RMSNorm gain and fused Q|K|V matrix (+bias) of the
 // single-token decode kernel that projects and attends in one launch.
 struct DecQkvIn {

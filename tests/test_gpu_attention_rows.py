@@ -1,0 +1,113 @@
+"""si_attention over batches of queries: the whole-row kernel (8 queries or
+more, 1, 2 or 4 KV groups) against 64 bits at the edges of its chunks and
+steps, with cache rows past each context poisoned, in contiguous and paged
+caches, and the per-group kernel where the workspace is the smaller one.
+
+Bound: fp16 hi + lo weights (2^-22), 32-bit sums over up to 2100 positions and
+the scores' rounding through the exponential, 1e-5 of a row's largest output."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import si_amd
+from tests.gpu_helpers import empty, host
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # qheads, kvheads, hdim, contexts
+    (28, 4, 128, [1, 2, 15, 16, 17, 63, 64, 65, 127, 128, 700, 2100]),
+    (14, 2, 64, [0, 1, 31, 32, 33, 128, 129, 999]),
+    (14, 2, 64, [5] * 8),
+    (12, 2, 128, [300, 1, 299, 0, 64, 65, 128, 300, 17]),
+    (5, 1, 32, [64, 63, 65, 1, 256, 257, 255, 0, 511]),
+    (16, 1, 96, [70, 1, 2, 3, 64, 65, 66, 100]),
+    (8, 4, 64, [40 + 7 * i for i in range(40)]),
+]
+
+
+def _want(q, k, v, ctx, per):
+    import torch
+    out = torch.zeros(q.shape, dtype=torch.float64, device="cuda")
+    for i, n in enumerate(ctx):
+        if n:
+            for h in range(q.shape[1]):
+                kg, vg = (t[i, :n, h // per].double() for t in (k, v))
+                p = (kg @ q[i, h].double() / q.shape[2] ** 0.5).softmax(0)
+                out[i, h] = p @ vg
+    return out
+
+
+def _check(out, want, ctx):
+    for i, n in enumerate(ctx):
+        if n == 0:
+            assert bool((out[i] == 0).all()), f"query {i}: empty context"
+            continue
+        err = (out[i].double() - want[i]).abs().amax(1) / want[i].abs().amax(1)
+        assert err.max().item() < 1e-5, (i, n, err.max().item())
+
+
+@pytest.mark.parametrize("qh,kv,d,ctx", CASES)
+def test_attention_rows_edges(qh, kv, d, ctx):
+    import torch
+    n, most = len(ctx), max(ctx)
+    g = torch.Generator(device="cuda").manual_seed(most)
+    q = torch.randn(n, qh, d, generator=g, device="cuda")
+    k, v = (torch.randn(n, most, kv, d, generator=g, device="cuda").half() for _ in range(2))
+    for i, c in enumerate(ctx):  # rows no context reaches
+        k[i, c:], v[i, c:] = float("nan"), float("inf")
+    want = _want(q, k, v, ctx, qh // kv)
+    s = si_amd.make_shape(32, qh, kv, d)
+    cd = torch.tensor(ctx, dtype=torch.int32, device="cuda")
+    full = si_amd.lib().si_attention_workspace(ctypes.byref(s), n, most)
+    per_group = max(1, min((512 + kv * n - 1) // (kv * n), (most + 63) // 64))
+    least = n * qh * max(per_group, 2) * (d + 2) * 4
+    results = []
+    for need in {full, min(full, least)}:
+        ws = torch.full((need // 4,), float("nan"), device="cuda")
+        out, qs = empty((n, qh, d), torch.float32), empty((n, qh * d), torch.int8)
+        sc = empty((n, qh * d // 32), torch.int16)
+        si_amd.call("si_attention", ctypes.byref(s), si_amd.ptr(q), n, si_amd.ptr(k),
+                    si_amd.ptr(v), k.stride(0), si_amd.ptr(cd), 0, 0, most, si_amd.ptr(out),
+                    si_amd.ptr(qs), si_amd.ptr(sc), None, si_amd.ptr(ws), need,
+                    si_amd.stream_handle())
+        _check(out, want, ctx)
+        results.append(out)
+    # the same rows through shuffled pages: the same bits as the contiguous call
+    page = 16
+    each = (most + page - 1) // page
+    table = torch.randperm(n * each, generator=g, device="cuda").to(torch.int32).view(n, each)
+    kp, vp = (torch.full((n * each, page, kv, d), float("nan"), device="cuda").half()
+              for _ in range(2))
+    pad = torch.full((n, each * page, kv, d), float("nan"), device="cuda").half()
+    for pool, t in ((kp, k), (vp, v)):
+        pad[:, :most] = t
+        pool[table.long().view(-1)] = pad.view(n * each, page, kv, d)
+    ws = torch.full((full // 4,), float("nan"), device="cuda")
+    out = empty((n, qh, d), torch.float32)
+    si_amd.call("si_attention_paged", ctypes.byref(s), si_amd.ptr(q), n, si_amd.ptr(kp),
+                si_amd.ptr(vp), n * each, page, si_amd.ptr(table), each, si_amd.ptr(cd), most,
+                si_amd.ptr(out), None, None, None, si_amd.ptr(ws), full, si_amd.stream_handle())
+    ws = torch.full((full // 4,), float("nan"), device="cuda")
+    flat = empty((n, qh, d), torch.float32)
+    si_amd.call("si_attention", ctypes.byref(s), si_amd.ptr(q), n, si_amd.ptr(k), si_amd.ptr(v),
+                k.stride(0), si_amd.ptr(cd), 0, 0, most, si_amd.ptr(flat), None, None, None,
+                si_amd.ptr(ws), full, si_amd.stream_handle())
+    assert np.array_equal(host(out), host(flat))
+
+
+def test_attention_rows_host_contexts():
+    """Contexts from the host (ctx0 + i * step, one cache per sequence)."""
+    import torch
+    qh, kv, d, n, ctx0, step = 14, 2, 64, 9, 30, 11
+    ctx = [ctx0 + step * i for i in range(n)]
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q = torch.randn(n, qh, d, generator=g, device="cuda")
+    k, v = (torch.randn(n, ctx[-1], kv, d, generator=g, device="cuda").half() for _ in range(2))
+    s = si_amd.make_shape(32, qh, kv, d)
+    need = si_amd.lib().si_attention_workspace(ctypes.byref(s), n, ctx[-1])
+    ws, out = empty((need,), torch.uint8), empty((n, qh, d), torch.float32)
+    si_amd.call("si_attention", ctypes.byref(s), si_amd.ptr(q), n, si_amd.ptr(k), si_amd.ptr(v),
+                k.stride(0), None, ctx0, step, ctx[-1], si_amd.ptr(out), None, None, None,
+                si_amd.ptr(ws), need, si_amd.stream_handle())
+    _check(out, _want(q, k, v, ctx, qh // kv), ctx)
