@@ -295,18 +295,22 @@ int si_ffn_gateup_q8(const float *h, const float *gain, int hidden, float eps,
 
 // SI_GEMM_F6 workspace: the fp6 weights w6 and scales d6, the activations
 // x6, then the K-split partials (none for the fused gate|up pass), each part
-// 256-byte aligned.
+// 256-byte aligned.  least: the same without room for the activations' scales
+// in x6 (what si_gemm_f6_workspace once asked for): from there to total the
+// call runs the default tile kernel, whose sums are the same bit for bit.
 struct F6Ws {
-    size_t w6 = 0, d6 = 0, x6 = 0, part = 0, total = 0;
+    size_t w6 = 0, d6 = 0, x6 = 0, part = 0, total = 0, least = 0;
 };
 static F6Ws f6_ws(int m, int n, int k, bool partials) {
     const size_t nb = (size_t)k / 32;
     const auto up = [](size_t b) { return (b + 255) / 256 * 256; };
     F6Ws o;
     o.d6 = up((size_t)n * nb * 24);
-    o.x6 = o.d6 + up((size_t)n * nb * 2);
-    o.part = o.x6 + up((size_t)m * nb * 48);
-    o.total = o.part + (partials ? up(gemm_f6_partial_bytes(m, n, k)) : 0);
+    o.x6 = o.d6 + up((size_t)f6_scale_rows(n) * nb * 2);
+    o.part = o.x6 + up(f6_x_bytes(m, (int)nb));
+    const size_t parts = partials ? up(gemm_f6_partial_bytes(m, n, k)) : 0;
+    o.total = o.part + parts;
+    o.least = o.d6 + up((size_t)n * nb * 2) + up((size_t)m * nb * 48) + parts;
     return o;
 }
 
@@ -334,14 +338,19 @@ int si_gemm_q4q8(const uint8_t *wqs, const uint16_t *wd, int tile, int n, int k,
                    "gemm: SI_GEMM_F6 operands beyond 2 GiB (m=%d n=%d k=%d)", m, n, k);
         if (m == 0) return SI_OK;
         const F6Ws L = f6_ws(m, n, k, true);
-        SI_REQUIRE(workspace && ws_bytes >= L.total && ((uintptr_t)workspace & 255) == 0,
+        SI_REQUIRE(workspace && ws_bytes >= L.least && ((uintptr_t)workspace & 255) == 0,
                    "gemm: SI_GEMM_F6 needs si_gemm_f6_workspace(m, n, k) = %zu bytes of "
                    "256-byte aligned workspace", L.total);
         uint8_t *ws = (uint8_t *)workspace;
         const hipStream_t st = S(stream);
+        if (ws_bytes < L.total) {
+            launch_gemm_q4q8(wqs, wd, tile, n, k, xqs, xd, m, bias, residual, out, ldo, false, ws,
+                             ws_bytes, st, true);
+            return check_launch("si_gemm_q4q8");
+        }
         launch_q4_to_w6(wqs, wd, n, k / 32, tile, 0, ws + L.w6, (uint16_t *)(ws + L.d6), st);
-        launch_q8_to_x6(xqs, m, k / 32, ws + L.x6, st);
-        launch_gemm_f6(ws + L.w6, (const uint16_t *)(ws + L.d6), n, k, ws + L.x6, xd, m, bias,
+        launch_q8_to_x6(xqs, xd, m, k / 32, ws + L.x6, st);
+        launch_gemm_f6(ws + L.w6, (const uint16_t *)(ws + L.d6), n, k, ws + L.x6, m, bias,
                        residual, out, ldo, ws + L.part, L.total - L.part, false, 0, nullptr,
                        nullptr, nullptr, nullptr, st);
         return check_launch("si_gemm_q4q8");
@@ -404,14 +413,19 @@ int si_gemm_gateup_q8(const uint8_t *wqs, const uint16_t *wd, int tile, int f, i
                    "gemm_gateup: SI_GEMM_F6 runs the fused one-pass plan only; this shape "
                    "splits K (m=%d f=%d k=%d)", m, f, k);
         const F6Ws L = f6_ws(m, 2 * f, k, false);
-        SI_REQUIRE(workspace && ws_bytes >= L.total && ((uintptr_t)workspace & 255) == 0,
+        SI_REQUIRE(workspace && ws_bytes >= L.least && ((uintptr_t)workspace & 255) == 0,
                    "gemm_gateup: SI_GEMM_F6 needs si_gemm_f6_workspace(m, 2f, k) = %zu bytes "
                    "of 256-byte aligned workspace", L.total);
         uint8_t *ws = (uint8_t *)workspace;
         const hipStream_t st = S(stream);
+        if (ws_bytes < L.total) {
+            launch_gemm_gateup_q8(wqs, wd, tile, f, k, xqs, xd, m, gu, act, qs, d, bsum, false,
+                                  nullptr, 0, st, false, nullptr, nullptr, nullptr, nullptr, true);
+            return check_launch("si_gemm_gateup_q8");
+        }
         launch_q4_to_w6(wqs, wd, 2 * f, k / 32, tile, f, ws + L.w6, (uint16_t *)(ws + L.d6), st);
-        launch_q8_to_x6(xqs, m, k / 32, ws + L.x6, st);
-        launch_gemm_f6(ws + L.w6, (const uint16_t *)(ws + L.d6), 2 * f, k, ws + L.x6, xd, m,
+        launch_q8_to_x6(xqs, xd, m, k / 32, ws + L.x6, st);
+        launch_gemm_f6(ws + L.w6, (const uint16_t *)(ws + L.d6), 2 * f, k, ws + L.x6, m,
                        nullptr, nullptr, gu, 2 * f, nullptr, 0, false, f, act, qs, d, bsum, st);
         return check_launch("si_gemm_gateup_q8");
     }
@@ -875,7 +889,7 @@ static int make_workspace(const si_shape_t *s, int max_tokens, int max_pos,
     TRY(m.alloc(&W->scores, (size_t)s->qheads * max_pos));
     // past 64 rows the gate|up GEMM (past 512 all four) runs in the fp6 formulation
     if (max_tokens > 64)
-        TRY(m.alloc(&W->x6, M * (size_t)(std::max(std::max(H, QD), F) / 32) * 48));
+        TRY(m.alloc(&W->x6, f6_x_bytes(max_tokens, std::max(std::max(H, QD), F) / 32)));
     // GEMM split-K partials: the largest need over the layer's projections
     // and every row count up to max_tokens (the split depends on both)
     {
@@ -974,7 +988,7 @@ static int upload_q4(DevArena &mem, Q4Dev *w, const std::vector<const uint8_t *>
 static int make_q6(DevArena &mem, const Q4Dev &q, int gu_f, Q6Dev *o) {
     const size_t cnt = (size_t)q.n * (q.k / 32);
     TRY(mem.alloc(&o->w, cnt * 24));
-    TRY(mem.alloc(&o->d, cnt));
+    TRY(mem.alloc(&o->d, (size_t)f6_scale_rows(q.n) * (q.k / 32)));
     launch_q4_to_w6(q.qs, q.d, q.n, q.k / 32, q.tile, gu_f, o->w, o->d, 0);
     HIP_TRY(hipDeviceSynchronize());
     return SI_OK;
@@ -1365,8 +1379,8 @@ static int run_rows(si_layer *L, const float *x, int rows, uint16_t *kc, uint16_
     if (roped)
         ;
     else if (f6) {
-        launch_q8_to_x6(L->xq.qs, rows, H / SI_QK, L->x6, st);
-        launch_gemm_f6(L->wqkv6.w, L->wqkv6.d, NQKV, H, L->x6, L->xq.d, rows, L->bqkv, nullptr,
+        launch_q8_to_x6(L->xq.qs, L->xq.d, rows, H / SI_QK, L->x6, st);
+        launch_gemm_f6(L->wqkv6.w, L->wqkv6.d, NQKV, H, L->x6, rows, L->bqkv, nullptr,
                        L->qkv, NQKV, L->gemm_ws, L->gemm_ws_bytes, false, 0, nullptr, nullptr,
                        nullptr, nullptr, st);
     } else if (tl_x && gemm_streams(rows, NQKV, H))
@@ -1426,8 +1440,8 @@ static int run_rows(si_layer *L, const float *x, int rows, uint16_t *kc, uint16_
         launch_gemm_q4q8_tiled(L->wo.qs, L->wo.d, L->wo.tile, L->wo.n, L->wo.k, L->attq.tq,
                                L->attq.td, rows, nullptr, nullptr, L->attn_out, L->wo.n, st);
     else if (f6) {
-        launch_q8_to_x6(L->attq.qs, rows, QD / SI_QK, L->x6, st);
-        osplits = launch_gemm_f6(L->wo6.w, L->wo6.d, L->wo.n, L->wo.k, L->x6, L->attq.d, rows,
+        launch_q8_to_x6(L->attq.qs, L->attq.d, rows, QD / SI_QK, L->x6, st);
+        osplits = launch_gemm_f6(L->wo6.w, L->wo6.d, L->wo.n, L->wo.k, L->x6, rows,
                                  nullptr, nullptr, L->attn_out, L->wo.n, L->gemm_ws,
                                  L->gemm_ws_bytes, true, 0, nullptr, nullptr, nullptr, nullptr,
                                  st);
@@ -1468,8 +1482,8 @@ static int run_rows(si_layer *L, const float *x, int rows, uint16_t *kc, uint16_
         // operand-tiled Q8 a streamed down projection reads)
         bool fused6 = false;
         if (f6gu) {
-            if (!norm_x6) launch_q8_to_x6(L->xq2.qs, rows, H / SI_QK, L->x6, st);
-            fused6 = launch_gemm_f6(L->wgu6.w, L->wgu6.d, 2 * s.ffn, H, L->x6, L->xq2.d, rows,
+            if (!norm_x6) launch_q8_to_x6(L->xq2.qs, L->xq2.d, rows, H / SI_QK, L->x6, st);
+            fused6 = launch_gemm_f6(L->wgu6.w, L->wgu6.d, 2 * s.ffn, H, L->x6, rows,
                                     nullptr, nullptr, capt(cap, L->gu), 2 * s.ffn, nullptr, 0,
                                     false, s.ffn, capt(cap, L->act), L->actq.qs, L->actq.d,
                                     L->actq.s, st, tiled ? L->actq.tq : nullptr,
@@ -1489,8 +1503,8 @@ static int run_rows(si_layer *L, const float *x, int rows, uint16_t *kc, uint16_
         launch_gemm_q4q8_tiled(L->wdown.qs, L->wdown.d, L->wdown.tile, H, s.ffn, L->actq.tq,
                                L->actq.td, rows, nullptr, L->h, out, H, st);
     else if (f6) {
-        launch_q8_to_x6(L->actq.qs, rows, s.ffn / SI_QK, L->x6, st);
-        launch_gemm_f6(L->wdown6.w, L->wdown6.d, H, s.ffn, L->x6, L->actq.d, rows, nullptr, L->h,
+        launch_q8_to_x6(L->actq.qs, L->actq.d, rows, s.ffn / SI_QK, L->x6, st);
+        launch_gemm_f6(L->wdown6.w, L->wdown6.d, H, s.ffn, L->x6, rows, nullptr, L->h,
                        out, H, L->gemm_ws, L->gemm_ws_bytes, false, 0, nullptr, nullptr, nullptr,
                        nullptr, st);
     } else

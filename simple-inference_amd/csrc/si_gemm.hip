@@ -568,6 +568,19 @@ __global__ void __launch_bounds__(256) k_gemm_fast(
 // that opens stage s and waited for (vmcnt(0)) before the next barrier, so it
 // overlaps a whole stage of matrix work, with one barrier per stage.  The
 // grid runs M tiles fastest (workgroups sharing a weight tile run together).
+// The scales come block-major with padded rows (f6_scale_rows), so a stage's
+// are two 16-byte copies; from the planar [m][nb] they were 8 of its 26
+// copies, 2 bytes a lane and a row apart: 633 -> 601 us for the 7B gate|up at
+// 2048 rows, 343 -> 312 for down, 113 -> 103 for Q|K|V.
+//
+// What bounds it: each tile and block needs ~74 cycles of the matrix pipe
+// (the dot and the scale product, ~37 each) and 16 fmas (~69), ~88 together
+// at best on two wavefronts; with live data the card then runs at ~1.8 GHz,
+// 48 ns of the 72 measured, the rest LDS reads and copies.  Measured and
+// not kept, all slower: operands of the next block read ahead into registers
+// with the fmas between the matrix instructions (671 us at 2 wavefronts per
+// SIMD, 647 at 3), 256 x 128 tiles (676), 2 wavefronts per SIMD (630); other
+// tile orders across the XCDs are within 2 %.
 // One lane's operand: 32 six-bit codes, bytes 0..15 at p16 (16-byte aligned)
 // and 16..23 at p8; the instruction reads six registers.
 __device__ __forceinline__ v8i f6_operand(const uint8_t *p16, const uint8_t *p8) {
@@ -589,7 +602,7 @@ __device__ __forceinline__ void f6_stage_sync() {
 template <int WM, int WN, int TM, int TN, bool FUSE>
 __global__ void __launch_bounds__(256, 3) k_gemm_f6(
     const uint8_t *__restrict__ w6, const uint16_t *__restrict__ d6, int n, int nb,
-    const uint8_t *__restrict__ x6, const uint16_t *__restrict__ xd, int m,
+    const uint8_t *__restrict__ x6, const uint16_t *__restrict__ xd6, int m,
     const float *__restrict__ bias, const float *__restrict__ residual, float *__restrict__ out,
     int ldo, float *__restrict__ part, int bps, GateUpOut go) {
     static_assert(!FUSE || TN == 2, "gate|up fusion pairs two column tiles per wavefront");
@@ -597,21 +610,20 @@ __global__ void __launch_bounds__(256, 3) k_gemm_f6(
     using C = GemmCfg<WM, WN, TM, TN>;
     constexpr int BM = C::BM, BN = C::BN;
     // a stage buffer: activations [G_KB][2] regions of BM rows, weights
-    // [G_KB] regions of BN rows (each [rows][16] then [rows][8]), scales x.d
-    // [G_KB][BM] and w.d [G_KB][BN] (fp16 bits zero-extended to a dword: the
-    // low register of the scale-product operand)
+    // [G_KB] regions of BN rows (each [rows][16] then [rows][8]), fp16 scales
+    // x.d [G_KB][BM] and w.d [G_KB][BN]
     constexpr int A_BYTES = G_KB * 2 * BM * F6_BYTES, B_BYTES = G_KB * BN * F6_BYTES;
-    constexpr int SX_OFF = A_BYTES + B_BYTES, SW_OFF = SX_OFF + G_KB * BM * 4;
-    constexpr int STAGE = SW_OFF + G_KB * BN * 4;
-    // wavefront copy instructions per stage: 64 lanes x 16 bytes (operands),
-    // 64 lanes x 2 bytes into dwords (scales); instruction q goes to
-    // wavefront q % 4
+    constexpr int SX_OFF = A_BYTES + B_BYTES, SW_OFF = SX_OFF + G_KB * BM * 2;
+    constexpr int STAGE = SW_OFF + G_KB * BN * 2;
+    // wavefront copy instructions per stage, 64 lanes x 16 bytes: instruction
+    // q goes to wavefront q % 4, the x.d and w.d copies (one each) to the
+    // next two
     constexpr int AR = BM * F6_BYTES / 16, BR = BN * F6_BYTES / 16;  // 16-byte pieces per region
     constexpr int A_WI = G_KB * 2 * AR / 64, B_WI = G_KB * BR / 64;
-    constexpr int SX_WI = G_KB * BM / 64, SW_WI = G_KB * BN / 64;
     static_assert(G_KB * 2 * AR % 64 == 0 && G_KB * BR % 64 == 0, "whole copy instructions");
+    static_assert(G_KB * BM <= 512 && G_KB * BN <= 512, "one copy instruction each");
     constexpr int A_PW = (A_WI + 3) / 4, B_PW = (B_WI + 3) / 4;
-    constexpr int SX_PW = (SX_WI + 3) / 4, SW_PW = (SW_WI + 3) / 4;
+    constexpr int SX_W = (A_WI + B_WI) % 4, SW_W = (A_WI + B_WI + 1) % 4;
     // sb0 also holds the gate|up epilogue's transposition
     constexpr int EPI = 4 * 32 * GEMM_EPI_FT * 4;
     __shared__ __attribute__((aligned(16))) uint8_t sb0[STAGE > EPI ? STAGE : EPI];
@@ -625,7 +637,7 @@ __global__ void __launch_bounds__(256, 3) k_gemm_f6(
     const int f6_sa = g ? 128 : 132;  // hi codes 2^5 (16 x the codes' 2^1), lo 2^1
 
     // stage-relative source offsets of this lane's copies
-    uint32_t oa[A_PW], ob[B_PW], osx[SX_PW], osw[SW_PW];
+    uint32_t oa[A_PW], ob[B_PW];
     // piece q of a region's stage slice: rows' 16-byte parts (q < rows),
     // then their 8-byte parts, in LDS at 16 q either way
 #pragma unroll
@@ -640,16 +652,9 @@ __global__ void __launch_bounds__(256, 3) k_gemm_f6(
         ob[i] = (uint32_t)(blk * n * F6_BYTES +
                            (q < BN ? n0 * 16 + q * 16 : n * 16 + n0 * 8 + (q - BN) * 16));
     }
-#pragma unroll
-    for (int i = 0; i < SX_PW; ++i) {
-        const int e = (4 * i + wave) * 64 + lane, blk = e / BM, row = e % BM;
-        osx[i] = (uint32_t)((min(m0 + row, m - 1) * nb + blk) * 2);
-    }
-#pragma unroll
-    for (int i = 0; i < SW_PW; ++i) {
-        const int e = (4 * i + wave) * 64 + lane, blk = e / BN, c = e % BN;
-        osw[i] = (uint32_t)((blk * n + min(n0 + c, n - 1)) * 2);
-    }
+    const uint32_t m8 = f6_scale_rows(m), n8 = f6_scale_rows(n);
+    const uint32_t osx = (lane / (BM / 8) * m8 + m0 + lane % (BM / 8) * 8) * 2;
+    const uint32_t osw = (lane / (BN / 8) * n8 + n0 + lane % (BN / 8) * 8) * 2;
     // copy the stage starting at block bs into buf: past row m or n a piece
     // reads the next region or, past the array, zero (buffer bounds); such
     // rows and columns reach only outputs that are never stored
@@ -660,8 +665,8 @@ __global__ void __launch_bounds__(256, 3) k_gemm_f6(
             buf_rsrc(x6 + (size_t)bs * 2 * m * F6_BYTES, left * 2 * (uint32_t)m * F6_BYTES);
         const __amdgpu_buffer_rsrc_t rb_s =
             buf_rsrc(w6 + (size_t)bs * n * F6_BYTES, left * (uint32_t)n * F6_BYTES);
-        const __amdgpu_buffer_rsrc_t rx_s = buf_rsrc(xd + bs, ((uint32_t)m * nb - bs) * 2);
-        const __amdgpu_buffer_rsrc_t rw_s = buf_rsrc(d6 + (size_t)bs * n, left * (uint32_t)n * 2);
+        const __amdgpu_buffer_rsrc_t rx_s = buf_rsrc(xd6 + (size_t)bs * m8, left * m8 * 2);
+        const __amdgpu_buffer_rsrc_t rw_s = buf_rsrc(d6 + (size_t)bs * n8, left * n8 * 2);
 #pragma unroll
         for (int i = 0; i < A_PW; ++i)
             if (A_WI % 4 == 0 || 4 * i + wu < A_WI)
@@ -670,14 +675,8 @@ __global__ void __launch_bounds__(256, 3) k_gemm_f6(
         for (int i = 0; i < B_PW; ++i)
             if (B_WI % 4 == 0 || 4 * i + wu < B_WI)
                 lds_copy16(rb_s, buf + A_BYTES + 1024 * (4 * i + wu), ob[i]);
-#pragma unroll
-        for (int i = 0; i < SX_PW; ++i)
-            if (SX_WI % 4 == 0 || 4 * i + wu < SX_WI)
-                lds_copy2(rx_s, buf + SX_OFF + 256 * (4 * i + wu), osx[i]);
-#pragma unroll
-        for (int i = 0; i < SW_PW; ++i)
-            if (SW_WI % 4 == 0 || 4 * i + wu < SW_WI)
-                lds_copy2(rw_s, buf + SW_OFF + 256 * (4 * i + wu), osw[i]);
+        if (wu == SX_W && lane < G_KB * BM / 8) lds_copy16(rx_s, buf + SX_OFF, osx);
+        if (wu == SW_W && lane < G_KB * BN / 8) lds_copy16(rw_s, buf + SW_OFF, osw);
     };
 
     float acc[TM][TN][16];
@@ -694,7 +693,7 @@ __global__ void __launch_bounds__(256, 3) k_gemm_f6(
     const int ra = wm * TM * 32 + j, rb = wn * TN * 32 + j;
     const int a16 = g * BM * F6_BYTES + ra * 16, a8 = g * BM * F6_BYTES + BM * 16 + ra * 8;
     const int b16 = A_BYTES + rb * 16, b8 = A_BYTES + BN * 16 + rb * 8;
-    const int sx_off = SX_OFF + ra * 4, sw_off = SW_OFF + rb * 4;
+    const int sx_off = SX_OFF + ra * 2, sw_off = SW_OFF + rb * 2;
     const auto compute = [&](const uint8_t *buf, int bs) {
 #pragma unroll
         for (int blk = 0; blk < G_KB; ++blk) {
@@ -710,7 +709,7 @@ __global__ void __launch_bounds__(256, 3) k_gemm_f6(
                 // keeps each operand's two reads its own (merged reads of two
                 // tiles' 8-byte parts cost register copies)
                 __builtin_amdgcn_sched_barrier(0);
-                const unsigned xs = *(const uint32_t *)(buf + sx_off + (blk * BM + a * 32) * 4);
+                const unsigned xs = *(const uint16_t *)(buf + sx_off + (blk * BM + a * 32) * 2);
                 asc[a] = __builtin_bit_cast(gh4, (v2u){xs, 0u});
             }
 #pragma unroll
@@ -718,7 +717,7 @@ __global__ void __launch_bounds__(256, 3) k_gemm_f6(
                 bop[b] = f6_operand(buf + b16 + blk * BN * F6_BYTES + b * 32 * 16,
                                     buf + b8 + blk * BN * F6_BYTES + b * 32 * 8);
                 __builtin_amdgcn_sched_barrier(0);
-                const unsigned ws = *(const uint32_t *)(buf + sw_off + (blk * BN + b * 32) * 4);
+                const unsigned ws = *(const uint16_t *)(buf + sw_off + (blk * BN + b * 32) * 2);
                 bsc[b] = __builtin_bit_cast(gh4, (v2u){g ? 0u : ws, 0u});
             }
 #pragma unroll
@@ -2014,7 +2013,7 @@ static void launch_bd(const BdPlan &p, int mode, const uint8_t *wqs, const uint1
 static int gemm_core(const uint8_t *wqs, const uint16_t *wd, int tile, int n, int k,
                      const int8_t *xqs, const uint16_t *xd, int m, const float *bias,
                      const float *residual, float *out, int ldo, bool exact, void *workspace,
-                     size_t ws_bytes, bool want_part, hipStream_t st);
+                     size_t ws_bytes, bool want_part, hipStream_t st, bool tile_only = false);
 
 int launch_gemm_q4q8_parts(const uint8_t *wqs, const uint16_t *wd, int tile, int n, int k,
                            const int8_t *xqs, const uint16_t *xd, int m, float *out, bool exact,
@@ -2034,9 +2033,9 @@ void launch_gemm_reduce(const float *part, int splits, int m, int n, float *out,
 void launch_gemm_q4q8(const uint8_t *wqs, const uint16_t *wd, int tile, int n, int k,
                       const int8_t *xqs, const uint16_t *xd, int m, const float *bias,
                       const float *residual, float *out, int ldo, bool exact, void *workspace,
-                      size_t ws_bytes, hipStream_t st) {
+                      size_t ws_bytes, hipStream_t st, bool tile_only) {
     gemm_core(wqs, wd, tile, n, k, xqs, xd, m, bias, residual, out, ldo, exact, workspace,
-              ws_bytes, false, st);
+              ws_bytes, false, st, tile_only);
 }
 
 void launch_gemm_q4q8_tiled(const uint8_t *wqs, const uint16_t *wd, int tile, int n, int k,
@@ -2080,7 +2079,7 @@ bool launch_gemm_qkv_rope(const uint8_t *wqs, const uint16_t *wd, int tile, int 
 static int gemm_core(const uint8_t *wqs, const uint16_t *wd, int tile, int n, int k,
                      const int8_t *xqs, const uint16_t *xd, int m, const float *bias,
                      const float *residual, float *out, int ldo, bool exact, void *workspace,
-                     size_t ws_bytes, bool want_part, hipStream_t st) {
+                     size_t ws_bytes, bool want_part, hipStream_t st, bool tile_only) {
     if (m <= 0 || n <= 0) return 0;
     const int nb = k / SI_QK;
     if (exact) {
@@ -2094,7 +2093,7 @@ static int gemm_core(const uint8_t *wqs, const uint16_t *wd, int tile, int n, in
     };
     float *part = nullptr;
     int splits;
-    if (bd_takes(m, n, nb)) {
+    if (!tile_only && bd_takes(m, n, nb)) {
         const BdPlan p = bd_plan(m, n, nb, 0);
         if (p.C == 1 || fits(p.C)) {
             part = p.C > 1 ? (float *)workspace : nullptr;
@@ -2163,8 +2162,11 @@ __device__ __forceinline__ void f6_store(uint8_t *p16, uint8_t *p8, const uint32
 // hi = q >> 4 (-8..7), then that of lo = q & 15 (q = 16 hi + lo), each m rows
 // as [m][16] then [m][8].  Grid (ceil(m / 64), nb), a thread per (row,
 // block), consecutive threads consecutive rows (one-wavefront workgroups: a
-// few hundred rows still spread over the CUs).
-__global__ void __launch_bounds__(64) k_q8_to_x6(const int8_t *__restrict__ qs, int m, int nb,
+// few hundred rows still spread over the CUs); then the scales, transposed to
+// [nb][f6_scale_rows(m)] (2-byte reads a row apart: +1..3 us at 2048 rows,
+// where the GEMM saves 20 % of its copy instructions, each a row apart too).
+__global__ void __launch_bounds__(64) k_q8_to_x6(const int8_t *__restrict__ qs,
+                                                 const uint16_t *__restrict__ d, int m, int nb,
                                                  uint8_t *__restrict__ x6) {
     const int row = blockIdx.x * 64 + threadIdx.x, blk = blockIdx.y;
     if (row >= m) return;
@@ -2180,12 +2182,13 @@ __global__ void __launch_bounds__(64) k_q8_to_x6(const int8_t *__restrict__ qs, 
     uint8_t *rh = x6 + (size_t)(2 * blk) * m * F6_BYTES, *rl = rh + (size_t)m * F6_BYTES;
     f6_store(rh + (size_t)row * 16, rh + (size_t)m * 16 + (size_t)row * 8, hi);
     f6_store(rl + (size_t)row * 16, rl + (size_t)m * 16 + (size_t)row * 8, lo);
+    f6_scales(x6, m, nb)[(size_t)blk * f6_scale_rows(m) + row] = d[(size_t)row * nb + blk];
 }
 
 // Repacked Q4 [nb][n][16] (byte i: element i low nibble, i + 16 high) and its
 // tiled scales -> w6 (per block a region of n rows, [n][16] then [n][8], codes
-// of nibble - 8: the two's-complement table at nibble ^ 8) and d6 [nb][n];
-// logical row r is physical row gate_up_row(r, gu_f) when gu_f > 0.
+// of nibble - 8: the two's-complement table at nibble ^ 8) and d6
+// [nb][f6_scale_rows(n)]; logical row r is physical row gate_up_row(r, gu_f) when gu_f > 0.
 __global__ void __launch_bounds__(256) k_q4_to_w6(const uint8_t *__restrict__ qs,
                                                   const uint16_t *__restrict__ d, int n, int nb,
                                                   int tile, int gu_f, uint8_t *__restrict__ w6,
@@ -2203,13 +2206,14 @@ __global__ void __launch_bounds__(256) k_q4_to_w6(const uint8_t *__restrict__ qs
     }
     uint8_t *rg = w6 + (size_t)blk * n * F6_BYTES;
     f6_store(rg + (size_t)r * 16, rg + (size_t)n * 16 + (size_t)r * 8, c);
-    d6[(size_t)blk * n + r] = d[q4_scale_index(pr, blk, nb, tile)];
+    d6[(size_t)blk * f6_scale_rows(n) + r] = d[q4_scale_index(pr, blk, nb, tile)];
 }
 
-void launch_q8_to_x6(const int8_t *qs, int m, int nb, uint8_t *x6, hipStream_t st) {
+void launch_q8_to_x6(const int8_t *qs, const uint16_t *d, int m, int nb, uint8_t *x6,
+                     hipStream_t st) {
     if (m <= 0 || nb <= 0) return;
-    SI_LAUNCH(k_q8_to_x6, dim3((unsigned)((m + 63) / 64), (unsigned)nb), dim3(64), 0, st, qs, m,
-              nb, x6);
+    SI_LAUNCH(k_q8_to_x6, dim3((unsigned)((m + 63) / 64), (unsigned)nb), dim3(64), 0, st, qs, d,
+              m, nb, x6);
 }
 
 void launch_q4_to_w6(const uint8_t *qs, const uint16_t *d, int n, int nb, int tile, int gu_f,
@@ -2225,7 +2229,7 @@ size_t gemm_f6_partial_bytes(int m, int n, int k) {
 }
 
 int launch_gemm_f6(const uint8_t *w6, const uint16_t *d6, int n, int k, const uint8_t *x6,
-                   const uint16_t *xd, int m, const float *bias, const float *residual,
+                   int m, const float *bias, const float *residual,
                    float *out, int ldo, void *workspace, size_t ws_bytes, bool want_part,
                    int gu_f, float *act, int8_t *aqs, uint16_t *ad, int16_t *as, hipStream_t st,
                    int8_t *atq, uint16_t *atd) {
@@ -2241,8 +2245,8 @@ int launch_gemm_f6(const uint8_t *w6, const uint16_t *d6, int n, int k, const ui
     const dim3 grid((m + p.bm - 1) / p.bm, (n + p.bn - 1) / p.bn, p.splits);
     const GateUpOut go{gu_f, act, aqs, ad, as, atq, atd};
 #define CALL(WM, WN, TM, TN, FUSE)                                                             \
-    SI_LAUNCH((k_gemm_f6<WM, WN, TM, TN, FUSE>), grid, dim3(256), 0, st, w6, d6, n, nb, x6, xd, \
-              m, bias, residual, out, ldo, part, p.bps, go)
+    SI_LAUNCH((k_gemm_f6<WM, WN, TM, TN, FUSE>), grid, dim3(256), 0, st, w6, d6, n, nb, x6,     \
+              f6_scales(x6, m, nb), m, bias, residual, out, ldo, part, p.bps, go)
     if (gu_f) {
         if (p.bm == 64)
             CALL(2, 2, 1, 2, true);
@@ -2277,7 +2281,7 @@ void launch_gemm_gateup_q8(const uint8_t *wqs, const uint16_t *wd, int tile, int
                            const int8_t *xqs, const uint16_t *xd, int m, float *gu, float *act,
                            int8_t *qs, uint16_t *d, int16_t *s, bool exact, void *workspace,
                            size_t ws_bytes, hipStream_t st, bool f16, int8_t *tq, uint16_t *td,
-                           const int8_t *txq, const uint16_t *txd) {
+                           const int8_t *txq, const uint16_t *txd, bool tile_only) {
     if (m <= 0) return;
     const int n = 2 * f, nb = k / SI_QK;
     if (f16 && !exact) {
@@ -2288,7 +2292,7 @@ void launch_gemm_gateup_q8(const uint8_t *wqs, const uint16_t *wd, int tile, int
                                      GateUpOut{f, act, qs, d, s, tq, td}, st);
         return;
     }
-    if (!exact && gateup_bd(m, k)) {
+    if (!exact && !tile_only && gateup_bd(m, k)) {
         // the activations streamed when given operand-tiled (txq / txd)
         const BdPlan p = bd_plan(m, n, nb, 1, txq && txd);
         launch_bd(p, 1, wqs, wd, tile, n, nb, p.da ? txq : xqs, p.da ? txd : xd, m, nullptr,
@@ -2299,7 +2303,7 @@ void launch_gemm_gateup_q8(const uint8_t *wqs, const uint16_t *wd, int tile, int
     // tile kernel's), or, with too little workspace, one pass into gu; then
     // the split reduce.  Without a split gemm_core would write gu, which is
     // optional here: the fused pass below.
-    const bool split = exact || gemm_splits(m, n, nb) > 1;
+    const bool split = exact || (!tile_only && gemm_splits(m, n, nb) > 1);
     if (split) {
         const int splits = gemm_core(wqs, wd, tile, n, k, xqs, xd, m, nullptr, nullptr, gu, n,
                                      exact, workspace, ws_bytes, true, st);

@@ -68,10 +68,11 @@ void launch_rmsnorm_q8_parts(const float *x, const float *part, int splits, cons
                              int rows, int n, float eps, float *y_out, float *h, float *normed,
                              int8_t *qs, uint16_t *d, int16_t *s, hipStream_t st,
                              int8_t *tq = nullptr, uint16_t *td = nullptr, uint8_t *x6 = nullptr);
+// tile_only: the tile kernel (k_gemm_fast) also where k_gemm_bd would run
 void launch_gemm_q4q8(const uint8_t *wqs, const uint16_t *wd, int tile, int n, int k,
                       const int8_t *xqs, const uint16_t *xd, int m, const float *bias,
                       const float *residual, float *out, int ldo, bool exact, void *workspace,
-                      size_t ws_bytes, hipStream_t st);
+                      size_t ws_bytes, hipStream_t st, bool tile_only = false);
 // planar Q8_0 (qs [m][k], d [m][k/32]) -> operand-tiled (q8_tiled_byte)
 void launch_q8_tile(const int8_t *qs, const uint16_t *d, int m, int k, int8_t *tq, uint16_t *td,
                     hipStream_t st);
@@ -90,7 +91,8 @@ void launch_gemm_gateup_q8(const uint8_t *wqs, const uint16_t *wd, int tile, int
                            int8_t *qs, uint16_t *d, int16_t *s, bool exact, void *workspace,
                            size_t ws_bytes, hipStream_t st, bool f16 = false,
                            int8_t *tq = nullptr, uint16_t *td = nullptr,
-                           const int8_t *txq = nullptr, const uint16_t *txd = nullptr);
+                           const int8_t *txq = nullptr, const uint16_t *txd = nullptr,
+                           bool tile_only = false);
 // Whether launch_gemm_gateup_q8 streams txq/txd (default flags) for m rows,
 // f features, K = k.
 bool gemm_gateup_streams(int m, int f, int k);
@@ -151,20 +153,34 @@ struct RopeOut {
 bool launch_gemm_qkv_rope(const uint8_t *wqs, const uint16_t *wd, int tile, int n, int k,
                           const int8_t *xqs, const uint16_t *xd, int m, const float *bias_perm,
                           float *out, const RopeOut &ro, hipStream_t st);
+// Rows of one block's fp16 scales in the fp6 operands: 16-byte aligned, so a
+// tile's scales are copied 16 bytes a lane.
+__host__ __device__ inline int f6_scale_rows(int rows) { return (rows + 7) & ~7; }
+__host__ __device__ inline uint16_t *f6_scales(uint8_t *x6, int m, int nb) {
+    return (uint16_t *)(x6 + (size_t)m * nb * 48);
+}
+__host__ __device__ inline const uint16_t *f6_scales(const uint8_t *x6, int m, int nb) {
+    return (const uint16_t *)(x6 + (size_t)m * nb * 48);
+}
+inline size_t f6_x_bytes(int m, int nb) {
+    return (size_t)m * nb * 48 + (size_t)f6_scale_rows(m) * nb * 2;
+}
 // The fp6 formulation of the fast-path GEMM (k_gemm_f6): the weights once as
-// w6 fp6 codes (n * nb * 24 bytes) + d6 [nb][n] fp16 scales (logical gate|up
-// row order when gu_f > 0), each Q8 activation as x6 (m * nb * 48 bytes: hi
-// and lo codes).  launch_gemm_f6 has gemm_core's plan, splits and reduce
+// w6 fp6 codes (n * nb * 24 bytes) + d6 [nb][f6_scale_rows(n)] fp16 scales
+// (logical gate|up row order when gu_f > 0), each Q8 activation as x6
+// (f6_x_bytes(m, nb): hi and lo codes, m * nb * 48 bytes, then the scales
+// [nb][f6_scale_rows(m)]).  launch_gemm_f6 has gemm_core's plan, splits and reduce
 // (want_part: the split count, partials left in the workspace); with gu_f > 0
 // it is the fused gate|up + SwiGLU + Q8 pass (out: the optional gate|up, ldo
 // 2 gu_f; atq/atd, optional: the Q8 also operand-tiled), and returns -1
 // (nothing launched) when that plan needs a K split.
-void launch_q8_to_x6(const int8_t *qs, int m, int nb, uint8_t *x6, hipStream_t st);
+void launch_q8_to_x6(const int8_t *qs, const uint16_t *d, int m, int nb, uint8_t *x6,
+                     hipStream_t st);
 size_t gemm_f6_partial_bytes(int m, int n, int k);  // launch_gemm_f6's K-split partials
 void launch_q4_to_w6(const uint8_t *qs, const uint16_t *d, int n, int nb, int tile, int gu_f,
                      uint8_t *w6, uint16_t *d6, hipStream_t st);
 int launch_gemm_f6(const uint8_t *w6, const uint16_t *d6, int n, int k, const uint8_t *x6,
-                   const uint16_t *xd, int m, const float *bias, const float *residual,
+                   int m, const float *bias, const float *residual,
                    float *out, int ldo, void *workspace, size_t ws_bytes, bool want_part,
                    int gu_f, float *act, int8_t *aqs, uint16_t *ad, int16_t *as, hipStream_t st,
                    int8_t *atq = nullptr, uint16_t *atd = nullptr);

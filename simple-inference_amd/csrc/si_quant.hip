@@ -220,7 +220,12 @@ __global__ void __launch_bounds__(T) k_rmsnorm_q8_v4(const float *__restrict__ x
                 *(uint32_t *)(tq + q8_tiled_byte(pb, r & 31, (4 * c) % SI_QK)) = packed;
                 if ((tid & 7) == 0) td[pb * 32 + (r & 31)] = dbits;
             }
-            if (x6) f6_store_oct(packed, x6, gridDim.x, r, (4 * c) / SI_QK);
+            if (x6) {
+                const int rows = gridDim.x, blk = (4 * c) / SI_QK;
+                f6_store_oct(packed, x6, rows, r, blk);
+                if ((tid & 7) == 0)
+                    f6_scales(x6, rows, n / SI_QK)[(size_t)blk * f6_scale_rows(rows) + r] = dbits;
+            }
         }
     }
 }
@@ -372,7 +377,7 @@ void launch_rmsnorm_q8(const float *x, const float *y, const float *gain, int ro
         SI_LAUNCH(k_rmsnorm_q8<false>, dim3(rows), dim3(256), lds, st, x, y, gain, n,
                   eps, h, normed, qs, d, s);
     if (tq) launch_q8_tile(qs, d, rows, n, tq, td, st);  // this path writes planar only
-    if (x6) launch_q8_to_x6(qs, rows, n / SI_QK, x6, st);
+    if (x6) launch_q8_to_x6(qs, d, rows, n / SI_QK, x6, st);
 }
 
 void launch_swiglu_q8(const float *gu, int rows, int f, float *act, int8_t *qs, uint16_t *d,
