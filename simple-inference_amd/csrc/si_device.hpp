@@ -314,7 +314,7 @@ __device__ __forceinline__ void quant_block_pair16(const float (&x)[16], uint32_
 // the hardware's 1 ulp; the quotient is the product with the reciprocal,
 // corrected by its remainder.  The same values as expf and the IEEE division
 // (rms 0.62, at most 3.1 halves of an ulp from 64 bits, both) without their
-// range checks: 18 instructions against about 30.
+// range checks: 19 instructions against about 30.
 __device__ __forceinline__ float swiglu(float g, float u) {
     const float gc = __builtin_amdgcn_fmed3f(g, -104.0f, 104.0f);  // e^-g is inf or 0 there
     const float t = __fmul_rn(gc, -1.44269502f), n = rintf(t);
@@ -322,10 +322,12 @@ __device__ __forceinline__ float swiglu(float g, float u) {
     lo = fmaf(gc, -1.92596303e-8f, lo);
     const float f = __fadd_rn(__fsub_rn(t, n), lo);
     const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
-    const float den = __fadd_rn(1.0f, e);
+    // both sides of the quotient over 4: the reciprocal of 1 + e^-g past 2^126
+    // would be subnormal, which the hardware gives as 0
+    const float g4 = __fmul_rn(0.25f, g), den = fmaf(0.25f, e, 0.25f);
     const float r = __builtin_amdgcn_rcpf(den);
-    const float q = __fmul_rn(g, r);
-    const float s = fmaf(fmaf(-den, q, g), r, q);
+    const float q = __fmul_rn(g4, r);
+    const float s = fmaf(fmaf(-den, q, g4), r, q);
     return __fmul_rn(s == s ? s : q, u);  // (den or g infinite: the remainder is NaN)
 }
 

@@ -51,8 +51,8 @@ def test_swiglu_range_edges():
     steps (e^-g, 1 + e^-g, the quotient, the product) bound the error by 4 * 2^-24 relative."""
     import torch
     f = 4096
-    g = np.concatenate([np.linspace(-87, 110, f - 8), [0.0, 1e-40, -1e-30, 88.8, 104, 1e30, -60,
-                                                       -86.9]]).astype(np.float32)
+    g = np.concatenate([np.linspace(-88.7, 110, f - 8), [0.0, 1e-40, -1e-30, 88.8, 104, 1e30, -88,
+                                                       -87.5]]).astype(np.float32)
     u = np.random.default_rng(3).normal(0, 1, f).astype(np.float32)
     act, qs, d = empty((f,), torch.float32), empty((f,), torch.int8), empty((f // QK,), torch.int16)
     si_amd.call("si_swiglu_q8", si_amd.ptr(dev(np.concatenate([g, u]))), 1, f, si_amd.ptr(act),
