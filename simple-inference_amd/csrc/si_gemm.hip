@@ -1230,12 +1230,20 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Workgroup id -> (row half h, K range c, slot s) with the halves of one
-// (c, s) on one XCD; q >= C * S: no work.
-__device__ __forceinline__ void bd_place(int id, int H, int S, int &h, int &q, int &c, int &s) {
+// Workgroup id -> (row half h, K range c, slot s); q >= C * S: no work.  The
+// halves of one (c, s) are on one XCD; packed (bd_plan): numbered through
+// the XCDs in turn instead, so only the slots at a border are on two.
+__device__ __forceinline__ void bd_place(int id, int H, int S, bool packed, int &h, int &q, int &c,
+                                         int &s) {
     const int x = id & 7, r = id >> 3;
-    h = r % H;
-    q = (r / H) * 8 + x;
+    if (packed) {
+        const int i = x * (int)(gridDim.x >> 3) + r;
+        h = i % H;
+        q = i / H;
+    } else {
+        h = r % H;
+        q = (r / H) * 8 + x;
+    }
     c = q / S;
     s = q - c * S;
 }
@@ -1245,8 +1253,8 @@ __global__ void __launch_bounds__(64 * BD_W) k_gemm_bd(
     const uint8_t *__restrict__ wqs, const uint16_t *__restrict__ wd, int tile, int n, int nb,
     const int8_t *__restrict__ xqs, const uint16_t *__restrict__ xd, int m,
     const float *__restrict__ bias, const float *__restrict__ residual, float *__restrict__ out,
-    int ldo, float *__restrict__ part, int H, int C, int S, int cb, int units, GateUpOut go,
-    RopeOut ro) {
+    int ldo, float *__restrict__ part, int H, int C, int S, int cb, int units, bool packed,
+    GateUpOut go, RopeOut ro) {
     static_assert(MODE == 1 ? TN == 2 : TN == 1, "MODE 0 and 2 take one tile, gate|up two");
     static_assert(BD_W >= 8 && BD_W <= 16 && BD_W % 4 == 0, "8, 12 or 16 wavefronts");
     static_assert(!PIPE || (TN == 1 && P % 2 == 0), "pipelined: one tile, an even unroll");
@@ -1260,7 +1268,7 @@ __global__ void __launch_bounds__(64 * BD_W) k_gemm_bd(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 31, g = lane >> 5;
     int h, q, c, s;
-    bd_place(blockIdx.x, H, S, h, q, c, s);
+    bd_place(blockIdx.x, H, S, !DA && packed, h, q, c, s);
     if (q >= C * S) return;  // the whole workgroup
     const int m0 = 32 * h, b0 = c * cb, len = min(nb, b0 + cb) - b0;
     const int k = nb * SI_QK;
@@ -1888,12 +1896,14 @@ static GemmPlan gemm_plan(int m, int n, int nb) {
 // workgroups (slots) per (half, range) sharing its tiles round robin, one
 // workgroup per CU (its LDS is most of the CU's).  Workgroup i runs on XCD
 // i % 8 and the H halves of a slot share one, so S is sized for at most 32
-// (one XCD's CUs) per XCD: C * S <= 8 * floor(32 / H).
+// (one XCD's CUs) per XCD: C * S <= 8 * floor(32 / H).  Staged activations
+// may be packed instead (bd_plan): C * S <= 256 / H, regardless of XCDs.
 constexpr int BD_SMALL_M = 64;  // every projection and the gate|up pair
 constexpr int BD_GU_W = 12;     // wavefronts of the gate|up instances
 constexpr int BD_MAX_M = 512;   // one-tile projections, when bd_takes() says so
 struct BdPlan {
     int H, C, S, cb, units, grid;
+    bool packed = false;  // bd_place
     bool da;  // streamed (operand-tiled) activations: one K range, no fill
     // streamed one-tile projection whose 32-row halves outnumber the CUs:
     // one unit per workgroup of 8 wavefronts, two workgroups per CU, so the
@@ -1901,6 +1911,9 @@ struct BdPlan {
     bool wide = false;
     size_t lds;
 };
+static int bd_xcd_slots(int H, int C, int units) {
+    return std::max(1, std::min(8 * std::max(1, 32 / H) / C, units));
+}
 static BdPlan bd_plan(int m, int n, int nb, int mode, bool da = false) {
     // (da: m <= 64; for mode 1 the caller keeps nb <= BD_MAX_CB as without)
     BdPlan p;
@@ -1909,13 +1922,24 @@ static BdPlan bd_plan(int m, int n, int nb, int mode, bool da = false) {
     p.C = da ? 1 : (nb + BD_MAX_CB - 1) / BD_MAX_CB;
     p.cb = (nb + p.C - 1) / p.C;
     p.units = mode == 1 ? n / 64 : (n + 31) / 32;
-    const int per_xcd = std::max(1, 32 / p.H);
-    p.S = std::max(1, std::min(8 * per_xcd / p.C, p.units));
+    p.S = bd_xcd_slots(p.H, p.C, p.units);
+    if (!da) {
+        // Halves that do not divide an XCD's 32 CUs leave up to 80 of the 256
+        // idle in slots of whole XCDs (11 halves: 2 slots, 22 CUs of 32).
+        // Slots are packed over all CUs where that shortens the walk; where
+        // it does not the added workgroups only fill (0.5B O, 333 rows: 2
+        // units either way, 7.8 -> 8.5 us).  us, before -> packed: 7B Q|K|V
+        // 333 rows 39.7 -> 34.0, O 32.4 -> 25.8, 384 rows 32.8 -> 29.9; 0.5B
+        // Q|K|V 333 rows 9.6 -> 8.4, down (two ranges) 16.6 -> 14.6.
+        const int s = std::max(1, std::min(256 / (p.H * p.C), p.units));
+        p.packed = (p.units + s - 1) / s < (p.units + p.S - 1) / p.S;
+        if (p.packed) p.S = s;
+    }
     if (da && mode == 0 && p.units * p.H > 256) {
         p.S = p.units;
         p.wide = true;
     }
-    p.grid = 8 * p.H * ((p.C * p.S + 7) / 8);
+    p.grid = p.packed ? (p.H * p.C * p.S + 7) / 8 * 8 : 8 * p.H * ((p.C * p.S + 7) / 8);
     p.lds = da ? (size_t)BD_RED : bd_lds(p.cb);
     if (da && mode == 1) {
         // k_gemm_bd's deferred gate|up epilogue: the wavefronts' partial
@@ -1941,7 +1965,9 @@ static bool bd_takes(int m, int n, int nb) {
     if (m <= BD_SMALL_M) return true;
     if (m > BD_MAX_M) return false;
     const BdPlan p = bd_plan(m, n, nb, 0);
-    return p.C <= 2 && (p.units + p.S - 1) / p.S * p.cb <= 1024;
+    // (in slots of whole XCDs, as measured)
+    const int S = bd_xcd_slots(p.H, p.C, p.units);
+    return p.C <= 2 && (p.units + S - 1) / S * p.cb <= 1024;
 }
 
 // K splits gemm_core plans for an m x n x nb problem (1: one pass, no
@@ -1976,7 +2002,7 @@ static void launch_bd(const BdPlan &p, int mode, const uint8_t *wqs, const uint1
         }                                                                                      \
         SI_LAUNCH((k_gemm_bd<TN, P, MODE, W, DA, PIPE>), dim3(p.grid), dim3(64 * W), p.lds,   \
                   st, wqs, wd, tile, n, nb, xqs, xd, m, bias, residual, out, ldo, part, p.H,   \
-                  p.C, p.S, p.cb, p.units, go, ro);                                            \
+                  p.C, p.S, p.cb, p.units, p.packed, go, ro);                                            \
     } while (0)
     // gate|up: 12 wavefronts (3 per SIMD; 4 weight blocks in flight fit
     // their registers); one tile: 16 (4 per SIMD, 7 of 112 blocks each, 4
