@@ -72,8 +72,17 @@ void launch_rope_kv(const float *qkv, int ldqkv, int ntok, int qheads, int kvhea
 
 constexpr int ATT_MAXPER = 16;  // query heads per KV group (the 16 MFMA columns)
 
+// Weight of a chunk whose running max is m under the head's max mx.  POW2: the
+// maxima are in powers of two (the decode kernels of si_decode.hip); otherwise
+// natural (k_attn_decode_mfma).  An empty chunk (m = -inf) weighs 0.
+template <bool POW2>
+__device__ __forceinline__ float part_weight(float m, float mx) {
+    return POW2 ? __builtin_amdgcn_exp2f(m - mx) : expf(m - mx);
+}
+
 // grid (qheads, nq), block hdim: merge chunks, normalise, quantize to Q8_0
 // (tq/td, optional: the Q8_0 also operand-tiled, q8_tiled_byte).
+template <bool POW2>
 __global__ void k_attn_combine(int qheads, int hdim, int nsplit, const float *__restrict__ ws_m,
                                const float *__restrict__ ws_l, const float *__restrict__ ws_o,
                                float *__restrict__ attn, int8_t *__restrict__ qs,
@@ -88,8 +97,8 @@ __global__ void k_attn_combine(int qheads, int hdim, int nsplit, const float *__
     float l = 0.0f, acc = 0.0f;
 #pragma unroll 8
     for (int s = 0; s < nsplit; ++s) {
-        // an empty chunk (m = -inf) weighs 0, and its output may be unwritten
-        const float ms = ws_m[base + s], w = __builtin_amdgcn_exp2f(ms - mx);
+        // (an empty chunk's output may be unwritten)
+        const float ms = ws_m[base + s], w = part_weight<POW2>(ms, mx);
         const float os = ws_o[(base + s) * hdim + jj];
         l = fmaf(ws_l[base + s], w, l);
         acc = fmaf(ms == -INFINITY ? 0.0f : os, w, acc);
@@ -140,6 +149,7 @@ __device__ __forceinline__ float block_reduce_1024(float v, float *red, bool is_
 // (group, column) merges the partials s = group, group + P, ... and the P
 // group sums are added in group order, so the loads of P partials are in
 // flight at once instead of one after another.
+template <bool POW2>
 __global__ __launch_bounds__(1024) void k_attn_combine_wide(
     int qheads, int hdim, int nsplit, const float *__restrict__ ws_m,
     const float *__restrict__ ws_l, const float *__restrict__ ws_o, float *__restrict__ attn,
@@ -157,8 +167,8 @@ __global__ __launch_bounds__(1024) void k_attn_combine_wide(
     float l = 0.0f, acc = 0.0f;
 #pragma unroll 4
     for (int s = grp; s < nsplit; s += P) {
-        // an empty chunk (m = -inf) weighs 0, and its output may be unwritten
-        const float ms = ws_m[base + s], w = __builtin_amdgcn_exp2f(ms - mx);
+        // (an empty chunk's output may be unwritten)
+        const float ms = ws_m[base + s], w = part_weight<POW2>(ms, mx);
         const float os = ws_o[(base + s) * hdim + jj];
         l = fmaf(ws_l[base + s], w, l);
         acc = fmaf(ms == -INFINITY ? 0.0f : os, w, acc);
@@ -194,16 +204,21 @@ __global__ __launch_bounds__(1024) void k_attn_combine_wide(
     }
 }
 
-// Either combine kernel by partial count.
-static void combine(int qheads, int hdim, int nq, int nsplit, const float *ws_m,
+// Either combine kernel by partial count, the maxima in powers of two or not.
+static void combine(int qheads, int hdim, int nq, int nsplit, bool pow2, const float *ws_m,
                     const float *ws_l, const float *ws_o, float *attn, int8_t *qs, uint16_t *d,
                     int16_t *bsum, hipStream_t st, int8_t *tq = nullptr, uint16_t *td = nullptr) {
-    if (nsplit >= 32)
-        SI_LAUNCH(k_attn_combine_wide, dim3(qheads, nq), dim3(1024 / hdim * hdim), 0, st,
-                  qheads, hdim, nsplit, ws_m, ws_l, ws_o, attn, qs, d, bsum, tq, td);
-    else
-        SI_LAUNCH(k_attn_combine, dim3(qheads, nq), dim3(hdim), 0, st, qheads, hdim,
-                  nsplit, ws_m, ws_l, ws_o, attn, qs, d, bsum, tq, td);
+#define CALL(KERNEL, BLOCK)                                                                      \
+    SI_LAUNCH(KERNEL, dim3(qheads, nq), dim3(BLOCK), 0, st, qheads, hdim, nsplit, ws_m, ws_l,    \
+              ws_o, attn, qs, d, bsum, tq, td)
+    if (nsplit >= 32) {
+        if (pow2) CALL(k_attn_combine_wide<true>, 1024 / hdim * hdim);
+        else CALL(k_attn_combine_wide<false>, 1024 / hdim * hdim);
+    } else {
+        if (pow2) CALL(k_attn_combine<true>, hdim);
+        else CALL(k_attn_combine<false>, hdim);
+    }
+#undef CALL
 }
 
 // ===========================================================================
@@ -227,6 +242,13 @@ static void combine(int qheads, int hdim, int nq, int nsplit, const float *ws_m,
 // j + 16*(i/4), register i%4.  The A/B operands give lane l row/column l%16
 // and the k-slice (l/16); A and B use the same k-slice per lane, so any
 // consistent assignment of reduction indices to slices is exact.
+//
+// It serves the calls whose results are few (dec_rows_ok's batches go to the
+// whole-row kernel): there one Q8_0 scale that falls to the other side of an
+// fp16 tie moves the result by more than 5e-5 of it, so the order of its sums
+// and its natural-exponent softmax are kept as they are.  In powers of two it
+// would take 0.1-0.4 us less of 5-8 at 2-7 queries of 256 positions, 0.1-1.5
+// of 5-24 at 4096.
 // ===========================================================================
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
@@ -245,7 +267,7 @@ template <int D>
 __global__ void __launch_bounds__(256) k_attn_decode_mfma(
     const float *__restrict__ q, int qheads, int kvheads, const uint16_t *__restrict__ kc,
     const uint16_t *__restrict__ vc, size_t kv_seq_stride, const int *__restrict__ ctx_dev,
-    int ctx0, int ctx_step, int max_ctx, int chunk, float scale2, float *__restrict__ ws_m,
+    int ctx0, int ctx_step, int max_ctx, int chunk, float scale, float *__restrict__ ws_m,
     float *__restrict__ ws_l, float *__restrict__ ws_o, KvPages pg, int kv_row) {
     constexpr int KS = D / 32;  // k-steps of the score MFMA
     constexpr int DT = D / 16;  // d-tiles of the PV MFMA
@@ -304,33 +326,30 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
             const int kpos = min(t0 + col, p1 - 1);
             const uint16_t *krow = kbase + pg.row(qi, kpos, kv_seq_stride, kvd) + 8 * grp;
             f4 sacc = (f4){0.f, 0.f, 0.f, 0.f};
-            h8 ka[KS];
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) ka[ks] = *(const h8 *)(krow + 32 * ks);
-            // the lo products first: they round at their own small magnitude
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-                sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], ql[ks], sacc, 0, 0, 0);
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-                sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], qh[ks], sacc, 0, 0, 0);
+            for (int ks = 0; ks < KS; ++ks) {
+                const uint4 kraw = *(const uint4 *)(krow + 32 * ks);
+                const h8 ka = __builtin_bit_cast(h8, kraw);
+                sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qh[ks], sacc, 0, 0, 0);
+                sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[ks], sacc, 0, 0, 0);
+            }
             // lane holds S^T[pos = t0 + 4*grp + r][head = col]
             float s[4];
             float mx = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int pos = t0 + 4 * grp + r;
-                s[r] = pos < p1 ? sacc[r] : -INFINITY;
+                s[r] = pos < p1 ? sacc[r] * scale : -INFINITY;
                 mx = fmaxf(mx, s[r]);
             }
             mx = fmaxf(mx, swap16_f(mx));
             mx = fmaxf(mx, swap32_f(mx));
-            const float mnew = fmaxf(m, mx * scale2);
-            const float alpha = __builtin_amdgcn_exp2f(m - mnew);  // 0 while m is -inf
+            const float mnew = fmaxf(m, mx);
+            const float alpha = expf(m - mnew);  // 0 while m is -inf
             float p[4], ps = 0.0f;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], scale2, -mnew));
+                p[r] = expf(s[r] - mnew);
                 ps += p[r];
             }
             ps += swap16_f(ps);
@@ -371,7 +390,7 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
     }
     __syncthreads();
     const float mall = fmaxf(fmaxf(mrg_m[0][col], mrg_m[1][col]), fmaxf(mrg_m[2][col], mrg_m[3][col]));
-    const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mall);  // a wave with no positions adds 0
+    const float w = m == -INFINITY ? 0.0f : expf(m - mall);  // a wave with no positions adds 0
     for (int k = 0; k < 4; ++k) {
         if (wave == k)
 #pragma unroll
@@ -388,7 +407,7 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
     if (wave == 0 && grp == 0 && col < per) {
         float l = 0.0f;
         for (int k = 0; k < 4; ++k)
-            if (mrg_m[k][col] != -INFINITY) l += mrg_l[k][col] * __builtin_amdgcn_exp2f(mrg_m[k][col] - mall);
+            if (mrg_m[k][col] != -INFINITY) l += mrg_l[k][col] * expf(mrg_m[k][col] - mall);
         ws_m[pbase + (size_t)col * nsplit] = mall;
         ws_l[pbase + (size_t)col * nsplit] = l;
     }
@@ -935,11 +954,11 @@ void launch_attention(const float *q, int nq, int qheads, int kvheads, int hdim,
     float *ws_m = (float *)workspace;
     float *ws_l = ws_m + (size_t)nq * qheads * ns;
     float *ws_o = ws_l + (size_t)nq * qheads * ns;
-    const float scale2 = softmax_scale2(hdim);
+    const float scale = 1.0f / sqrtf((float)hdim);  // attention_kernels.h:86
     const dim3 grid(ns, kvheads, nq);
 #define SI_ATTN_LAUNCH(DIM)                                                                  \
     SI_LAUNCH(k_attn_decode_mfma<DIM>, grid, dim3(256), 0, st, q, qheads, kvheads, kc,       \
-              vc, kv_seq_stride, ctx_dev, ctx0, ctx_step, max_ctx, chunk, scale2, ws_m,      \
+              vc, kv_seq_stride, ctx_dev, ctx0, ctx_step, max_ctx, chunk, scale, ws_m,       \
               ws_l, ws_o, pg, kv_row)
     switch (hdim) {
         case 32: SI_ATTN_LAUNCH(32); break;
@@ -948,18 +967,19 @@ void launch_attention(const float *q, int nq, int qheads, int kvheads, int hdim,
         default: SI_ATTN_LAUNCH(128); break;
     }
 #undef SI_ATTN_LAUNCH
-    combine(qheads, hdim, nq, ns, ws_m, ws_l, ws_o, attn, qs, d, bsum, st);
+    combine(qheads, hdim, nq, ns, false, ws_m, ws_l, ws_o, attn, qs, d, bsum, st);
 }
 
-// Merge of nsplit partials laid out as [nq][qheads][nsplit] (m, l) and
-// [nq][qheads][nsplit][hdim] (o) in one workspace.
+// Merge of nsplit partials of the decode kernels (m in powers of two) laid out
+// as [nq][qheads][nsplit] (m, l) and [nq][qheads][nsplit][hdim] (o) in one
+// workspace.
 void launch_attn_combine(int nq, int qheads, int hdim, int nsplit, const void *workspace,
                          float *attn, int8_t *qs, uint16_t *d, int16_t *bsum, hipStream_t st,
                          int8_t *tq, uint16_t *td) {
     const float *ws_m = (const float *)workspace;
     const float *ws_l = ws_m + (size_t)nq * qheads * nsplit;
     const float *ws_o = ws_l + (size_t)nq * qheads * nsplit;
-    combine(qheads, hdim, nq, nsplit, ws_m, ws_l, ws_o, attn, qs, d, bsum, st, tq, td);
+    combine(qheads, hdim, nq, nsplit, true, ws_m, ws_l, ws_o, attn, qs, d, bsum, st, tq, td);
 }
 
 // ---------------------------------------------------------------------------

@@ -194,9 +194,9 @@ void launch_rope_kv(const float *qkv, int ldqkv, int ntok, int qheads, int kvhea
                     int pos0, int pos_step, int max_pos, const int *ctx_dev, const float *rc,
                     const float *rs, float *q_out, uint16_t *kc, uint16_t *vc,
                     size_t kv_seq_stride, hipStream_t st, KvPages pg = KvPages());
-// The attention kernels' softmax runs in powers of two: exp(s / sqrt(hdim))
-// (attention_kernels.h:86) = 2^(s * softmax_scale2), and the running maxima of
-// every partial state (ws_m) are in that scale.
+// The softmax of the prefill kernel and of si_decode.hip's runs in powers of
+// two: exp(s / sqrt(hdim)) (attention_kernels.h:86) = 2^(s * softmax_scale2),
+// and the running maxima of their partial states (ws_m) are in that scale.
 inline float softmax_scale2(int hdim) { return 1.44269504088896340736f / sqrtf((float)hdim); }
 int attn_nsplit(int kvheads, int nq, int max_ctx);
 // Partial states of launch_attention: what it runs best with, and the least

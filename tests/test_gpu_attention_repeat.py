@@ -1,0 +1,67 @@
+"""si_attention's per-group kernel gives the bytes it has always given: callers
+compare runs across versions, and over a few hundred Q8_0 scales a single one
+next to an fp16 tie moves the whole result by more than 5e-5 of it.
+
+The digests are those of the library as first optimised (natural-exponent
+softmax, hi and lo products interleaved): SHA-256 over the fp32 output, the Q8_0
+values, scales and block sums."""
+import ctypes
+import hashlib
+
+import numpy as np
+import pytest
+
+import si_amd
+from tests.gpu_helpers import dev, empty, host
+
+pytestmark = pytest.mark.gpu
+
+# qheads, kvheads, hdim, contexts, max_ctx, page size (0: contiguous) -> digest
+CASES = [
+    (14, 2, 64, [129, 1, 0, 333], 333, 0, "5cb0bab873b2297c"),
+    (12, 2, 128, [1283, 1332], 1332, 0, "45a819dc0ba9708b"),
+    (28, 4, 128, [64, 65, 700, 63, 16, 17, 1], 700, 16, "2154c418be02ba25"),
+    (5, 1, 32, [2200], 2200, 0, "ae9e73f1a7200f95"),
+    (16, 1, 96, [40, 255, 256, 257], 300, 64, "791e77d6631622ed"),
+]
+
+
+def digest(qh, kv, d, ctx, max_ctx, page):
+    import torch
+    n = len(ctx)
+    rng = np.random.default_rng([qh, kv, d, max_ctx, n])
+    q = dev(rng.standard_normal((n, qh, d)).astype(np.float32))
+    k, v = (rng.standard_normal((n, max_ctx, kv, d)).astype(np.float16) for _ in range(2))
+    s = si_amd.make_shape(32, qh, kv, d)
+    c = dev(np.array(ctx, np.int32))
+    need = si_amd.lib().si_attention_workspace(ctypes.byref(s), n, max_ctx)
+    ws = empty((need,), torch.uint8)
+    out, qs = empty((n, qh * d), torch.float32), empty((n, qh * d), torch.int8)
+    sc, bs = (empty((n, qh * d // 32), torch.int16) for _ in range(2))
+    outs = [si_amd.ptr(t) for t in (out, qs, sc, bs)]
+    p, st = si_amd.ptr, si_amd.stream_handle()
+    if page:
+        each = -(-max_ctx // page)
+        table = rng.permutation(n * each).astype(np.int32).reshape(n, each)
+        pools = []
+        for t in (k, v):
+            pad = np.zeros((n, each * page, kv, d), np.float16)
+            pad[:, :max_ctx] = t
+            pool = np.zeros((n * each, page, kv, d), np.float16)
+            pool[table.reshape(-1)] = pad.reshape(n * each, page, kv, d)
+            pools.append(dev(pool))
+        si_amd.call("si_attention_paged", ctypes.byref(s), p(q), n, p(pools[0]), p(pools[1]),
+                    n * each, page, p(dev(table)), each, p(c), max_ctx, *outs, p(ws), need, st)
+    else:
+        k, v = dev(k), dev(v)
+        si_amd.call("si_attention", ctypes.byref(s), p(q), n, p(k), p(v), k.stride(0), p(c), 0, 0,
+                    max_ctx, *outs, p(ws), need, st)
+    h = hashlib.sha256()
+    for t in (out, qs, sc, bs):
+        h.update(host(t).tobytes())
+    return h.hexdigest()[:16]
+
+
+@pytest.mark.parametrize("qh,kv,d,ctx,max_ctx,page,want", CASES)
+def test_same_bytes(qh, kv, d, ctx, max_ctx, page, want):
+    assert digest(qh, kv, d, ctx, max_ctx, page) == want
