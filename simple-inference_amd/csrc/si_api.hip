@@ -1288,9 +1288,6 @@ static int run_decode(si_layer *L, const float *x, uint16_t *kc, uint16_t *vc, i
     }
     // :272-275: Q8 of the attention output, W_O (no bias); + x in the full layer
     mark(L, SI_PHASE_OUT_PROJ, st);
-    const float *pm = (const float *)L->attn_ws;
-    const float *pl = pm + (size_t)s.qheads * ns;
-    const float *po = pl + (size_t)s.qheads * ns;
     if ((size_t)s.qheads * ns * (s.hdim + 2) * sizeof(float) > 32 * 1024) {
         // many chunk partials (7B at long contexts): merge them once instead
         // of in every W_O workgroup (each would re-read all of them)
@@ -1300,8 +1297,9 @@ static int run_decode(si_layer *L, const float *x, uint16_t *kc, uint16_t *vc, i
                       nullptr, full ? x : nullptr, full ? L->h : out, exact, st,
                       full ? capt(cap, L->attn_out) : nullptr);
     } else {
-        launch_dec_wo(pm, pl, po, ns, s.qheads, s.hdim, L->wo.qs, L->wo.d, L->wo.tile, H,
-                      full ? x : nullptr, capt(cap, L->attn), capt(cap, L->attq.qs),
+        launch_dec_wo(AttnParts(L->attn_ws, (size_t)s.qheads * ns, s.hdim), ns, s.qheads, s.hdim,
+                      L->wo.qs, L->wo.d, L->wo.tile, H, full ? x : nullptr,
+                      capt(cap, L->attn), capt(cap, L->attq.qs),
                       capt(cap, L->attq.d), capt(cap, L->attq.s),
                       full ? capt(cap, L->attn_out) : nullptr, full ? L->h : out, exact, st);
     }

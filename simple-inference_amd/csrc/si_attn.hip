@@ -205,12 +205,12 @@ __global__ __launch_bounds__(1024) void k_attn_combine_wide(
 }
 
 // Either combine kernel by partial count, the maxima in powers of two or not.
-static void combine(int qheads, int hdim, int nq, int nsplit, bool pow2, const float *ws_m,
-                    const float *ws_l, const float *ws_o, float *attn, int8_t *qs, uint16_t *d,
-                    int16_t *bsum, hipStream_t st, int8_t *tq = nullptr, uint16_t *td = nullptr) {
+static void combine(int qheads, int hdim, int nq, int nsplit, bool pow2, const AttnParts &pt,
+                    float *attn, int8_t *qs, uint16_t *d, int16_t *bsum, hipStream_t st,
+                    int8_t *tq = nullptr, uint16_t *td = nullptr) {
 #define CALL(KERNEL, BLOCK)                                                                      \
-    SI_LAUNCH(KERNEL, dim3(qheads, nq), dim3(BLOCK), 0, st, qheads, hdim, nsplit, ws_m, ws_l,    \
-              ws_o, attn, qs, d, bsum, tq, td)
+    SI_LAUNCH(KERNEL, dim3(qheads, nq), dim3(BLOCK), 0, st, qheads, hdim, nsplit, pt.m, pt.l,    \
+              pt.o, attn, qs, d, bsum, tq, td)
     if (nsplit >= 32) {
         if (pow2) CALL(k_attn_combine_wide<true>, 1024 / hdim * hdim);
         else CALL(k_attn_combine_wide<false>, 1024 / hdim * hdim);
@@ -951,15 +951,13 @@ void launch_attention(const float *q, int nq, int qheads, int kvheads, int hdim,
     const int ns = attn_nsplit(kvheads, nq, max_ctx);
     int chunk = (max_ctx + ns - 1) / ns;
     chunk = (chunk + MA_SUPER - 1) / MA_SUPER * MA_SUPER;
-    float *ws_m = (float *)workspace;
-    float *ws_l = ws_m + (size_t)nq * qheads * ns;
-    float *ws_o = ws_l + (size_t)nq * qheads * ns;
+    const AttnParts pt(workspace, (size_t)nq * qheads * ns, hdim);
     const float scale = 1.0f / sqrtf((float)hdim);  // attention_kernels.h:86
     const dim3 grid(ns, kvheads, nq);
 #define SI_ATTN_LAUNCH(DIM)                                                                  \
     SI_LAUNCH(k_attn_decode_mfma<DIM>, grid, dim3(256), 0, st, q, qheads, kvheads, kc,       \
-              vc, kv_seq_stride, ctx_dev, ctx0, ctx_step, max_ctx, chunk, scale, ws_m,       \
-              ws_l, ws_o, pg, kv_row)
+              vc, kv_seq_stride, ctx_dev, ctx0, ctx_step, max_ctx, chunk, scale, pt.m,       \
+              pt.l, pt.o, pg, kv_row)
     switch (hdim) {
         case 32: SI_ATTN_LAUNCH(32); break;
         case 64: SI_ATTN_LAUNCH(64); break;
@@ -967,19 +965,16 @@ void launch_attention(const float *q, int nq, int qheads, int kvheads, int hdim,
         default: SI_ATTN_LAUNCH(128); break;
     }
 #undef SI_ATTN_LAUNCH
-    combine(qheads, hdim, nq, ns, false, ws_m, ws_l, ws_o, attn, qs, d, bsum, st);
+    combine(qheads, hdim, nq, ns, false, pt, attn, qs, d, bsum, st);
 }
 
-// Merge of nsplit partials of the decode kernels (m in powers of two) laid out
-// as [nq][qheads][nsplit] (m, l) and [nq][qheads][nsplit][hdim] (o) in one
-// workspace.
-void launch_attn_combine(int nq, int qheads, int hdim, int nsplit, const void *workspace,
+// Merge of the decode kernels' nsplit partials per query and head (m in powers
+// of two).
+void launch_attn_combine(int nq, int qheads, int hdim, int nsplit, void *workspace,
                          float *attn, int8_t *qs, uint16_t *d, int16_t *bsum, hipStream_t st,
                          int8_t *tq, uint16_t *td) {
-    const float *ws_m = (const float *)workspace;
-    const float *ws_l = ws_m + (size_t)nq * qheads * nsplit;
-    const float *ws_o = ws_l + (size_t)nq * qheads * nsplit;
-    combine(qheads, hdim, nq, nsplit, true, ws_m, ws_l, ws_o, attn, qs, d, bsum, st, tq, td);
+    const AttnParts pt(workspace, (size_t)nq * qheads * nsplit, hdim);
+    combine(qheads, hdim, nq, nsplit, true, pt, attn, qs, d, bsum, st, tq, td);
 }
 
 // ---------------------------------------------------------------------------

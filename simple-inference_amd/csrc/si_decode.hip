@@ -1281,14 +1281,14 @@ void launch_dec_qkv(const float *x, const float *gain, int hidden, float eps, co
 #undef CALL
 }
 
-void launch_dec_wo(const float *pm, const float *pl, const float *po, int ns, int qheads,
-                   int hdim, const uint8_t *wqs, const uint16_t *wd, int tile, int n,
-                   const float *residual, float *cap_attn, int8_t *cap_qs, uint16_t *cap_d,
-                   int16_t *cap_s, float *cap_y, float *out, bool exact, hipStream_t st) {
+void launch_dec_wo(const AttnParts &pt, int ns, int qheads, int hdim, const uint8_t *wqs,
+                   const uint16_t *wd, int tile, int n, const float *residual, float *cap_attn,
+                   int8_t *cap_qs, uint16_t *cap_d, int16_t *cap_s, float *cap_y, float *out,
+                   bool exact, hipStream_t st) {
     const int qd = qheads * hdim;
 #define CALL(R, T, E)                                                                            \
     SI_LAUNCH((k_dec_wo<R, T, E>), dim3((n + R - 1) / R), dim3(T),                               \
-              (DecLds<R, T>::bytes(qd, false, 0)), st, pm, pl, po, ns,                           \
+              (DecLds<R, T>::bytes(qd, false, 0)), st, pt.m, pt.l, pt.o, ns,                     \
               qheads, hdim, wqs, wd, tile, n, residual, cap_attn, cap_qs, cap_d, cap_s,          \
               cap_y, out)
     if (exact) {
@@ -1407,9 +1407,7 @@ static void dec_attn_impl(const float *qkv, int ldqkv, int nq, int qheads, int k
     if (nq <= 0) return;
     int chunk = (max_ctx + ns - 1) / ns;
     chunk = (chunk + DA_TILE - 1) / DA_TILE * DA_TILE;
-    float *ws_m = (float *)workspace;
-    float *ws_l = ws_m + (size_t)nq * qheads * ns;
-    float *ws_o = ws_l + (size_t)nq * qheads * ns;
+    const AttnParts pt(workspace, (size_t)nq * qheads * ns, hdim);
     const float scale2 = softmax_scale2(hdim);
     const int per = qheads / kvheads;
     const bool fin = attn != nullptr;
@@ -1426,8 +1424,8 @@ static void dec_attn_impl(const float *qkv, int ldqkv, int nq, int qheads, int k
         }                                                                                         \
         SI_LAUNCH((k_dec_attn_rows<DIM, GG, FIN, PAGED, false>), dim3(ns, nq), dim3(256),         \
                   (RowsLds<DIM, GG>::bytes(per)), st, qkv, ldqkv, qheads, rc, rs, kc, vc,         \
-                  kv_seq_stride, ctx_dev, ctx0, max_ctx, chunk, scale2, q_cap, ws_m, ws_l,         \
-                  ws_o, attn, aqs, ad, as, pg, 0);                                                \
+                  kv_seq_stride, ctx_dev, ctx0, max_ctx, chunk, scale2, q_cap, pt.m, pt.l,         \
+                  pt.o, attn, aqs, ad, as, pg, 0);                                                \
     } while (0)
 #define RCALLG(DIM)                                                \
     if (kvheads == 1) {                                            \
@@ -1452,7 +1450,7 @@ static void dec_attn_impl(const float *qkv, int ldqkv, int nq, int qheads, int k
     SI_LAUNCH((k_dec_attn<DIM, NW, FIN, PAGED, DEP>), grid, dim3(NW * 64),                     \
               (AttnLds<DIM, NW>::bytes(per)), st, qkv, ldqkv, qheads, kvheads, rc, rs,         \
               kc, vc, kv_seq_stride, ctx_dev, ctx0, max_ctx, chunk, scale2, q_cap,              \
-              ws_m, ws_l, ws_o, attn, aqs, ad, as, pg, DecQkvIn{})
+              pt.m, pt.l, pt.o, attn, aqs, ad, as, pg, DecQkvIn{})
 #define CALLN(DIM, NW, FIN)                                             \
     if (chunk <= DA_TILE * NW) {                                        \
         CALL(DIM, NW, FIN, 1);                                          \
@@ -1495,9 +1493,7 @@ static void attn_rows_impl(const float *q, int nq, int qheads, int kvheads, int 
                            const int *ctx_dev, int ctx0, int ctx_step, int max_ctx, int ns,
                            void *workspace, hipStream_t st, KvPages pg) {
     const int chunk = ((max_ctx + ns - 1) / ns + DA_TILE - 1) / DA_TILE * DA_TILE;
-    float *ws_m = (float *)workspace;
-    float *ws_l = ws_m + (size_t)nq * qheads * ns;
-    float *ws_o = ws_l + (size_t)nq * qheads * ns;
+    const AttnParts pt(workspace, (size_t)nq * qheads * ns, hdim);
     const float scale2 = softmax_scale2(hdim);
     const int per = qheads / kvheads;
 #define RCALL(DIM, GG)                                                                           \
@@ -1513,7 +1509,7 @@ static void attn_rows_impl(const float *q, int nq, int qheads, int kvheads, int 
         SI_LAUNCH((k_dec_attn_rows<DIM, GG, false, PAGED, true>), dim3(ns, nq), dim3(256),       \
                   (RowsLds<DIM, GG>::bytes(per)), st, q, qheads *hdim, qheads, nullptr, nullptr, \
                   const_cast<uint16_t *>(kc), const_cast<uint16_t *>(vc), kv_seq_stride,         \
-                  ctx_dev, ctx0, max_ctx, chunk, scale2, nullptr, ws_m, ws_l, ws_o, nullptr,      \
+                  ctx_dev, ctx0, max_ctx, chunk, scale2, nullptr, pt.m, pt.l, pt.o, nullptr,      \
                   nullptr, nullptr, nullptr, pg, ctx_step);                                      \
     } while (0)
 #define RCALLG(DIM)                      \
@@ -1562,9 +1558,7 @@ void launch_dec_qkv_attn(const DecQkvIn &fq, int qheads, int kvheads, int hdim, 
                          float *q_cap, void *workspace, hipStream_t st) {
     int chunk = (ctx + ns - 1) / ns;
     chunk = (chunk + DA_TILE - 1) / DA_TILE * DA_TILE;
-    float *ws_m = (float *)workspace;
-    float *ws_l = ws_m + (size_t)qheads * ns;
-    float *ws_o = ws_l + (size_t)qheads * ns;
+    const AttnParts pt(workspace, (size_t)qheads * ns, hdim);
     const float scale2 = softmax_scale2(hdim);
     const dim3 grid(ns, qheads, 1);
 #define FQCALL(DIM, DEP)                                                                       \
@@ -1572,7 +1566,7 @@ void launch_dec_qkv_attn(const DecQkvIn &fq, int qheads, int kvheads, int hdim, 
               ((AttnLds<DIM, DA_NW>::bytes(1) + 15) / 16 * 16 +                                \
                FqLds<DIM, DA_NW>::bytes(fq.hidden)),                                           \
               st, nullptr, 0, qheads, kvheads, rc, rs, kc, vc, (size_t)0, nullptr, ctx, ctx,   \
-              chunk, scale2, q_cap, ws_m, ws_l, ws_o, nullptr, nullptr, nullptr, nullptr,       \
+              chunk, scale2, q_cap, pt.m, pt.l, pt.o, nullptr, nullptr, nullptr, nullptr,       \
               KvPages(), fq)
     const bool one = chunk <= DA_TILE * DA_NW;
     if (hdim == 64) {

@@ -198,6 +198,15 @@ void launch_rope_kv(const float *qkv, int ldqkv, int ntok, int qheads, int kvhea
 // two: exp(s / sqrt(hdim)) (attention_kernels.h:86) = 2^(s * softmax_scale2),
 // and the running maxima of their partial states (ws_m) are in that scale.
 inline float softmax_scale2(int hdim) { return 1.44269504088896340736f / sqrtf((float)hdim); }
+// The n partial states ([query][head][chunk]) of an attention in a workspace of
+// n * (hdim + 2) floats: the unnormalised outputs o [n][hdim], then the running
+// maxima m [n] and sums l [n].  o comes first: it is stored and read 16 bytes
+// a lane, and behind m and l it would be 8-byte aligned for odd n.
+struct AttnParts {
+    float *o, *m, *l;
+    AttnParts(void *ws, size_t n, int hdim)
+        : o((float *)ws), m(o + n * (size_t)hdim), l(m + n) {}
+};
 int attn_nsplit(int kvheads, int nq, int max_ctx);
 // Partial states of launch_attention: what it runs best with, and the least
 // it takes (fewer, longer context chunks).
@@ -225,10 +234,10 @@ void launch_dec_qkv(const float *x, const float *gain, int hidden, float eps, co
                     const uint16_t *wd, int tile, int n, const float *bias, float *cap_normed,
                     int8_t *cap_qs, uint16_t *cap_d, int16_t *cap_s, float *qkv, bool exact,
                     hipStream_t st);
-void launch_dec_wo(const float *pm, const float *pl, const float *po, int ns, int qheads,
-                   int hdim, const uint8_t *wqs, const uint16_t *wd, int tile, int n,
-                   const float *residual, float *cap_attn, int8_t *cap_qs, uint16_t *cap_d,
-                   int16_t *cap_s, float *cap_y, float *out, bool exact, hipStream_t st);
+void launch_dec_wo(const AttnParts &pt, int ns, int qheads, int hdim, const uint8_t *wqs,
+                   const uint16_t *wd, int tile, int n, const float *residual, float *cap_attn,
+                   int8_t *cap_qs, uint16_t *cap_d, int16_t *cap_s, float *cap_y, float *out,
+                   bool exact, hipStream_t st);
 void launch_dec_gateup(const float *h, const float *gain, int hidden, float eps,
                        const uint8_t *wqs, const uint16_t *wd, int tile, int f,
                        float *cap_normed,
@@ -271,7 +280,7 @@ void launch_dec_attn(const float *qkv, int ldqkv, int nq, int qheads, int kvhead
                      float *q_cap, int ns, void *workspace, float *attn, int8_t *aqs,
                      uint16_t *ad, int16_t *as, hipStream_t st, KvPages pg = KvPages());
 // tq/td (optional): the Q8_0 also operand-tiled (q8_tiled_byte; qs required)
-void launch_attn_combine(int nq, int qheads, int hdim, int nsplit, const void *workspace,
+void launch_attn_combine(int nq, int qheads, int hdim, int nsplit, void *workspace,
                          float *attn, int8_t *qs, uint16_t *d, int16_t *bsum, hipStream_t st,
                          int8_t *tq = nullptr, uint16_t *td = nullptr);
 // Kernels over the reference's own formats (si_mirror.hip): row-major Q4_0

@@ -23,6 +23,7 @@ CASES = [  # qheads, kvheads, hdim, contexts
     (5, 1, 32, [64, 63, 65, 1, 256, 257, 255, 0, 511]),
     (16, 1, 96, [70, 1, 2, 3, 64, 65, 66, 100]),
     (8, 4, 64, [40 + 7 * i for i in range(40)]),
+    (5, 1, 32, [200, 1, 17, 64, 0, 199, 128, 2, 65]),  # an odd count of partial states
 ]
 
 
