@@ -243,8 +243,8 @@ static void combine(int qheads, int hdim, int nq, int nsplit, bool pow2, const A
 // and the k-slice (l/16); A and B use the same k-slice per lane, so any
 // consistent assignment of reduction indices to slices is exact.
 //
-// It serves the calls whose results are few (dec_rows_ok's batches go to the
-// whole-row kernel): there one Q8_0 scale that falls to the other side of an
+// It serves the calls whose results are few (large batches go to the whole-row
+// kernel, attn_rows_nsplit): there one Q8_0 scale that falls to the other side of an
 // fp16 tie moves the result by more than 5e-5 of it, so the order of its sums
 // and its natural-exponent softmax are kept as they are.  In powers of two it
 // would take 0.1-0.4 us less of 5-8 at 2-7 queries of 256 positions, 0.1-1.5
@@ -902,18 +902,29 @@ size_t attn_workspace_min(int qheads, int hdim, int kvheads, int nq, int max_ctx
     return (size_t)nq * qheads * ns * (hdim + 2) * sizeof(float);
 }
 
-// Context chunks of the whole-row kernel for si_attention's queries (0: not
-// its shape, the per-group kernel runs): at least four steps each, about 512
-// workgroups in all (two per CU; workgroups past a query's context leave at
-// once), no more than 31 (32 take the wide merge: 4.4 -> 8-10 us), and
-// partials within 16 MB or the per-group kernel's.  Measured (us, kernel +
-// merge; per-group kernel -> this, 512 | 1024 workgroups aimed at): 48 queries
-// x 200-4096 positions (7B heads) 104.7 + 4.1 -> 51.5 + 4.5 | 50.9 + 6.9; 64 x
-// 4096 157 + 4.2 -> 94.8 + 4.2 | 98.3 + 4.5; 20 x 1000-4000 43.7 + 4.4 -> 19.9 +
-// 4.4 | 24 + 9; 0.5B heads, 64 x 10-4000 35.5 + 4.1 -> 18.2 + 4.1, 24 x 100-2048
-// 11.8 + 4.0 -> 7.6 + 4.0; 8 x 1-300 (7B) 9.4 + 4.0 -> 7.4 + 4.0.
+// Context chunks of the whole-row kernel for si_attention's queries (0: the
+// per-group kernel runs: not the shape, or caches below ROWS_CACHE): chunks of
+// about four steps, about 512 workgroups in all (two per CU; workgroups past a
+// query's context leave at once), no more than 31 (32 take the wide merge:
+// 4.4 -> 8-10 us), and partials within 16 MB or the per-group kernel's.
+// Measured (us, kernel + merge; per-group kernel -> this, 512 | 1024 workgroups
+// aimed at): 48 queries x 200-4096 positions (7B heads) 104.7 + 4.1 -> 51.5 + 4.5
+// | 50.9 + 6.9; 64 x 4096 157 + 4.2 -> 94.8 + 4.2 | 98.3 + 4.5; 20 x 1000-4000
+// 43.7 + 4.4 -> 19.9 + 4.4 | 24 + 9; 0.5B heads, 64 x 10-4000 35.5 + 4.1 -> 18.2
+// + 4.1.
+//
+// ROWS_CACHE, over the K and V rows of nq contexts of max_ctx: below it the call
+// is its two launches by either kernel (us a call, per-group -> this: 0.5B heads
+// 8 x 64-1024 12.1 -> 12.4, 16 x 1024, 8.4 MB, 12.3 -> 12.4; 12 heads of 128, 8
+// x 1024, 8.4 MB, 12.3 -> 12.6; 7B 8 x 256 12.3 -> 12.5), and its results are
+// few, where a scale that falls to the other side of an fp16 tie moves them by
+// more than 5e-5: they stay the per-group kernel's.  Above: 12 heads of 128, 10 x
+// 1024, 10.5 MB, 13.8 -> 12.4; 0.5B 24 x 1024, 12.6 MB, 13.6 -> 12.4; 7B 24 x 256,
+// 12.6 MB, 15.0 -> 11.5.
+constexpr size_t ROWS_CACHE = (size_t)10 << 20;
 static int attn_rows_nsplit(int qheads, int kvheads, int hdim, int nq, int max_ctx) {
     if (!dec_rows_ok(qheads, kvheads, hdim, nq)) return 0;
+    if ((size_t)nq * max_ctx * kvheads * hdim * 4 < ROWS_CACHE) return 0;
     const int rows = 16 * (4 / kvheads);
     const int ns = min((max_ctx + 4 * rows - 1) / (4 * rows), (512 + nq - 1) / nq);
     const size_t each = (size_t)nq * qheads * (hdim + 2) * sizeof(float);

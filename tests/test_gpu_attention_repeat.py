@@ -1,5 +1,5 @@
-"""si_attention's per-group kernel gives the bytes it has always given: callers
-compare runs across versions, and over a few hundred Q8_0 scales a single one
+"""si_attention over a few queries, or over little cache, gives the bytes it has
+always given (the per-group kernel's): callers compare runs across versions, and over a few hundred Q8_0 scales a single one
 next to an fp16 tie moves the whole result by more than 5e-5 of it.
 
 The digests are those of the library as first optimised (natural-exponent
@@ -23,6 +23,10 @@ CASES = [
     (28, 4, 128, [64, 65, 700, 63, 16, 17, 1], 700, 16, "2154c418be02ba25"),
     (5, 1, 32, [2200], 2200, 0, "ae9e73f1a7200f95"),
     (16, 1, 96, [40, 255, 256, 257], 300, 64, "791e77d6631622ed"),
+    (14, 2, 64, [80, 49, 64, 65, 1, 0, 70, 79, 63, 50, 77], 80, 0, "ba8c9b40af9b33e6"),
+    (28, 4, 128, [256, 1, 17, 200, 64, 128, 129, 255], 256, 0, "228747668c665a18"),
+    (12, 2, 128, [9, 1000, 500, 63, 999, 2, 700, 300], 1000, 16, "693b1329d44b589a"),
+    (5, 1, 32, [200, 1, 17, 64, 0, 199, 128, 2, 65], 200, 0, "504a78c534b5326d"),
 ]
 
 

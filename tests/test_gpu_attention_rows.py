@@ -1,7 +1,8 @@
 """si_attention over batches of queries: the whole-row kernel (8 queries or
-more, 1, 2 or 4 KV groups) against 64 bits at the edges of its chunks and
-steps, with cache rows past each context poisoned, in contiguous and paged
-caches, and the per-group kernel where the workspace is the smaller one.
+more, 1, 2 or 4 KV groups, 10 MiB of cache rows or more) against 64 bits at the
+edges of its chunks and steps, with cache rows past each context poisoned, in
+contiguous and paged caches, and the per-group kernel where the caches or the
+workspace are smaller.
 
 Bound: fp16 hi + lo weights (2^-22), 32-bit sums over up to 2100 positions and
 the scores' rounding through the exponential, 1e-5 of a row's largest output."""
@@ -15,7 +16,7 @@ from tests.gpu_helpers import empty, host
 
 pytestmark = pytest.mark.gpu
 
-CASES = [  # qheads, kvheads, hdim, contexts
+CASES = [  # qheads, kvheads, hdim, contexts (the longest is max_ctx)
     (28, 4, 128, [1, 2, 15, 16, 17, 63, 64, 65, 127, 128, 700, 2100]),
     (14, 2, 64, [0, 1, 31, 32, 33, 128, 129, 999]),
     (14, 2, 64, [5] * 8),
@@ -23,8 +24,15 @@ CASES = [  # qheads, kvheads, hdim, contexts
     (5, 1, 32, [64, 63, 65, 1, 256, 257, 255, 0, 511]),
     (16, 1, 96, [70, 1, 2, 3, 64, 65, 66, 100]),
     (8, 4, 64, [40 + 7 * i for i in range(40)]),
-    (5, 1, 32, [200, 1, 17, 64, 0, 199, 128, 2, 65]),  # an odd count of partial states
+    (5, 1, 32, [200, 1, 17, 64, 0, 199, 128, 2, 65]),
+    # past ROWS_CACHE, contexts about the chunks' ends
+    (28, 4, 128, [1, 63, 64, 65, 127, 129, 700, 0]),        # 11 chunks of 64
+    (14, 2, 64, [0, 1, 127, 128, 129, 256, 257, 31, 2304]),  # 18 of 128
+    (12, 2, 128, [1200, 1, 0, 127, 128, 129, 160, 31, 1199]),
+    (5, 1, 32, [9300, 1, 303, 304, 305, 63, 64, 65, 0]),  # an odd count of partial states
+    (16, 1, 96, [3500, 1, 255, 256, 257, 64, 65, 2]),
 ]
+ROWS_CACHE = 10 << 20  # bytes of K and V rows from which the whole-row kernel runs
 
 
 def _want(q, k, v, ctx, per):
@@ -63,17 +71,17 @@ def test_attention_rows_edges(qh, kv, d, ctx):
     full = si_amd.lib().si_attention_workspace(ctypes.byref(s), n, most)
     per_group = max(1, min((512 + kv * n - 1) // (kv * n), (most + 63) // 64))
     least = n * qh * max(per_group, 2) * (d + 2) * 4
-    results = []
     for need in {full, min(full, least)}:
         ws = torch.full((need // 4,), float("nan"), device="cuda")
         out, qs = empty((n, qh, d), torch.float32), empty((n, qh * d), torch.int8)
         sc = empty((n, qh * d // 32), torch.int16)
-        si_amd.call("si_attention", ctypes.byref(s), si_amd.ptr(q), n, si_amd.ptr(k),
-                    si_amd.ptr(v), k.stride(0), si_amd.ptr(cd), 0, 0, most, si_amd.ptr(out),
-                    si_amd.ptr(qs), si_amd.ptr(sc), None, si_amd.ptr(ws), need,
-                    si_amd.stream_handle())
+        ran = si_amd.kernel_times_ms("k_", lambda: si_amd.call(
+            "si_attention", ctypes.byref(s), si_amd.ptr(q), n, si_amd.ptr(k), si_amd.ptr(v),
+            k.stride(0), si_amd.ptr(cd), 0, 0, most, si_amd.ptr(out), si_amd.ptr(qs),
+            si_amd.ptr(sc), None, si_amd.ptr(ws), need, si_amd.stream_handle()))
+        rows = need == full and n * most * kv * d * 4 >= ROWS_CACHE
+        assert ran[0][0].startswith("k_dec_attn_rows" if rows else "k_attn_decode_mfma"), ran
         _check(out, want, ctx)
-        results.append(out)
     # the same rows through shuffled pages: the same bits as the contiguous call
     page = 16
     each = (most + page - 1) // page
