@@ -70,3 +70,25 @@ def test_swiglu_range_edges():
     got = host(act)[:5]
     assert got[0] == 0 and got[1] == 0 and np.isnan(got[2]) and got[3] == np.inf and \
         np.isnan(got[4])
+
+
+def test_swiglu_small_gates():
+    """silu(g) = g / 2 for |g| below 2^-60, rounded once: subnormal gates, those a
+    quarter of which is subnormal, and zeros of either sign, bit for bit."""
+    import torch
+    bits = np.concatenate([np.arange(1, 64), 1 << np.arange(23), (1 << np.arange(23)) + 1,
+                           [0x7fffff], np.arange(1, 66) * 0x800000, np.arange(1, 66) * 0x800000 + 1,
+                           np.arange(1, 66) * 0x800000 + 0x7fffff]).astype(np.uint32)
+    bits = np.concatenate([bits, bits | 0x80000000, [0, 0x80000000]]).astype(np.uint32)
+    g = np.resize(bits, (len(bits) + QK - 1) // QK * QK).view(np.float32)
+    for scale in (np.float32(1), np.float32(2.0 ** 100), np.float32(-1.5 * 2.0 ** 90)):
+        u = np.full_like(g, scale)
+        f = len(g)
+        act, qs, d = (empty((k,), t) for k, t in ((f, torch.float32), (f, torch.int8),
+                                                  (f // QK, torch.int16)))
+        si_amd.call("si_swiglu_q8", si_amd.ptr(dev(np.concatenate([g, u]))), 1, f, si_amd.ptr(act),
+                    si_amd.ptr(qs), si_amd.ptr(d), None, si_amd.stream_handle())
+        want = (g.astype(np.float64) / 2).astype(np.float32) * u
+        got = host(act)
+        bad = got.view(np.uint32) != want.view(np.uint32)
+        assert not bad.any(), [(float(x).hex(), y, z) for x, y, z in zip(g[bad][:4], got[bad], want[bad])]
