@@ -824,8 +824,12 @@ k_attn_prefill(const float *__restrict__ q, int ntok, int qheads, int kvheads, i
 
 // Causal prefill of ntok tokens at positions pos0.. of one sequence whose
 // cache rows 0..pos0+ntok-1 are in place (RoPE'd K, V).
-bool attn_prefill_supported(int qheads, int kvheads, int hdim) {
-    return kvheads > 0 && qheads % kvheads == 0 && qheads / kvheads <= 16 &&
+// The tiles are copied 16 bytes a lane straight into LDS, which takes aligned
+// rows (a row is a multiple of 64 bytes): a cache at any other address goes to
+// launch_attention's kernels, whose plain loads take it.
+bool attn_prefill_supported(int qheads, int kvheads, int hdim, const uint16_t *kc,
+                            const uint16_t *vc) {
+    return (((uintptr_t)kc | (uintptr_t)vc) & 15) == 0 && kvheads > 0 && qheads % kvheads == 0 && qheads / kvheads <= 16 &&
            (hdim == 32 || hdim == 64 || hdim == 96 || hdim == 128);
 }
 
