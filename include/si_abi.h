@@ -153,10 +153,14 @@ int si_q4q8_block_dots(const uint8_t *wqs, const uint16_t *wd, int n, int k,
  * 32 x 32 tile and block gives the block's integer dot exactly, as a float
  * (no conversion in the epilogue).  The call converts both operands into
  * the workspace first, which must be si_gemm_f6_workspace(m, n, k) bytes
- * (gate|up: n = 2f), 256-byte aligned.  The sums are those of the default
- * tile kernel's plan (bit for bit where the default runs it: more than 512
- * rows, or a shape the streaming kernel does not take).  No reference
- * counterpart: a device formulation of matvec_q4q8 (qwen_one_layer.c:148-162). */
+ * (gate|up: n = 2f), 256-byte aligned.  A workspace without room for the
+ * activations' scales (m rounded up to 8, times k/32 * 2 bytes: what that
+ * function left out when it was first published) is taken too, and the call
+ * then runs the default int8 tile kernel: the same bits, at its speed.  The
+ * sums are those of the default tile kernel's plan (bit for bit where the
+ * default runs it: more than 512 rows, or a shape the streaming kernel does
+ * not take).  No reference counterpart: a device formulation of matvec_q4q8
+ * (qwen_one_layer.c:148-162). */
 enum { SI_GEMM_EXACT = 1, SI_GEMM_F16 = 2, SI_GEMM_TILED_A = 4, SI_GEMM_F6 = 8 };
 
 /* Operand-tiled Q8_0 (the activation operand of SI_GEMM_TILED_A): rows in

@@ -340,7 +340,8 @@ int si_gemm_q4q8(const uint8_t *wqs, const uint16_t *wd, int tile, int n, int k,
         const F6Ws L = f6_ws(m, n, k, true);
         SI_REQUIRE(workspace && ws_bytes >= L.least && ((uintptr_t)workspace & 255) == 0,
                    "gemm: SI_GEMM_F6 needs si_gemm_f6_workspace(m, n, k) = %zu bytes of "
-                   "256-byte aligned workspace", L.total);
+                   "256-byte aligned workspace (the default tile kernel, from %zu on)",
+                   L.total, L.least);
         uint8_t *ws = (uint8_t *)workspace;
         const hipStream_t st = S(stream);
         if (ws_bytes < L.total) {
@@ -415,7 +416,8 @@ int si_gemm_gateup_q8(const uint8_t *wqs, const uint16_t *wd, int tile, int f, i
         const F6Ws L = f6_ws(m, 2 * f, k, false);
         SI_REQUIRE(workspace && ws_bytes >= L.least && ((uintptr_t)workspace & 255) == 0,
                    "gemm_gateup: SI_GEMM_F6 needs si_gemm_f6_workspace(m, 2f, k) = %zu bytes "
-                   "of 256-byte aligned workspace", L.total);
+                   "of 256-byte aligned workspace (the default tile kernel, from %zu on)",
+                   L.total, L.least);
         uint8_t *ws = (uint8_t *)workspace;
         const hipStream_t st = S(stream);
         if (ws_bytes < L.total) {
