@@ -1414,14 +1414,9 @@ static void dec_attn_impl(const float *qkv, int ldqkv, int nq, int qheads, int k
     if (dec_rows_ok(qheads, kvheads, hdim, nq)) {
 #define RCALL(DIM, GG, FIN)                                                                       \
     do {                                                                                          \
-        static bool big_lds = false;                                                              \
-        if (!big_lds) {                                                                           \
-            /* past 64 KB of dynamic LDS; a failure surfaces as the launch's error */            \
-            (void)hipFuncSetAttribute((const void *)k_dec_attn_rows<DIM, GG, FIN, PAGED, false>,  \
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,                 \
-                                      (int)ROWS_LDS_MAX);                                         \
-            big_lds = true;                                                                       \
-        }                                                                                         \
+        static PerDevice big_lds;                                                                 \
+        allow_lds(big_lds, (const void *)k_dec_attn_rows<DIM, GG, FIN, PAGED, false>,             \
+                  (int)ROWS_LDS_MAX);                                                             \
         SI_LAUNCH((k_dec_attn_rows<DIM, GG, FIN, PAGED, false>), dim3(ns, nq), dim3(256),         \
                   (RowsLds<DIM, GG>::bytes(per)), st, qkv, ldqkv, qheads, rc, rs, kc, vc,         \
                   kv_seq_stride, ctx_dev, ctx0, max_ctx, chunk, scale2, q_cap, pt.m, pt.l,         \
@@ -1498,14 +1493,9 @@ static void attn_rows_impl(const float *q, int nq, int qheads, int kvheads, int 
     const int per = qheads / kvheads;
 #define RCALL(DIM, GG)                                                                           \
     do {                                                                                         \
-        static bool big_lds = false;                                                             \
-        if (!big_lds) {                                                                          \
-            /* past 64 KB of dynamic LDS; a failure surfaces as the launch's error */           \
-            (void)hipFuncSetAttribute((const void *)k_dec_attn_rows<DIM, GG, false, PAGED, true>, \
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,                \
-                                      (int)ROWS_LDS_MAX);                                        \
-            big_lds = true;                                                                      \
-        }                                                                                        \
+        static PerDevice big_lds;                                                                \
+        allow_lds(big_lds, (const void *)k_dec_attn_rows<DIM, GG, false, PAGED, true>,           \
+                  (int)ROWS_LDS_MAX);                                                            \
         SI_LAUNCH((k_dec_attn_rows<DIM, GG, false, PAGED, true>), dim3(ns, nq), dim3(256),       \
                   (RowsLds<DIM, GG>::bytes(per)), st, q, qheads *hdim, qheads, nullptr, nullptr, \
                   const_cast<uint16_t *>(kc), const_cast<uint16_t *>(vc), kv_seq_stride,         \

@@ -1849,14 +1849,8 @@ static void launch_h16(dim3 grid, const uint8_t *wqs, const uint16_t *wd, int ti
                        const float *residual, float *out, int ldo, float *part, int bps,
                        const GateUpOut &go, hipStream_t st) {
     using C = H16Cfg<WM, WN, TM, TN>;
-    static bool big_lds = false;
-    if (!big_lds) {
-        // a failure here surfaces as the launch's error
-        (void)hipFuncSetAttribute((const void *)k_gemm_h16<WM, WN, TM, TN, FUSE>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)C::lds_bytes());
-        big_lds = true;
-    }
+    static PerDevice big_lds;
+    allow_lds(big_lds, (const void *)k_gemm_h16<WM, WN, TM, TN, FUSE>, (int)C::lds_bytes());
     SI_LAUNCH((k_gemm_h16<WM, WN, TM, TN, FUSE>), grid, dim3(C::NT), C::lds_bytes(), st, wqs, wd,
               tile, n, nb, xqs, xd, m, bias, residual, out, ldo, part, bps, go);
 }
@@ -1993,16 +1987,11 @@ static void launch_bd(const BdPlan &p, int mode, const uint8_t *wqs, const uint1
                       const GateUpOut &go, hipStream_t st, const RopeOut &ro = RopeOut{}) {
 #define BD(TN, P, MODE, W, DA, PIPE)                                                           \
     do {                                                                                       \
-        static bool big_lds = false;                                                           \
-        if (!big_lds) {                                                                        \
-            /* a failure here surfaces as the launch's error */                                \
-            (void)hipFuncSetAttribute((const void *)k_gemm_bd<TN, P, MODE, W, DA, PIPE>,       \
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, BD_LDS_MAX); \
-            big_lds = true;                                                                    \
-        }                                                                                      \
+        static PerDevice big_lds;                                                              \
+        allow_lds(big_lds, (const void *)k_gemm_bd<TN, P, MODE, W, DA, PIPE>, BD_LDS_MAX);     \
         SI_LAUNCH((k_gemm_bd<TN, P, MODE, W, DA, PIPE>), dim3(p.grid), dim3(64 * W), p.lds,   \
                   st, wqs, wd, tile, n, nb, xqs, xd, m, bias, residual, out, ldo, part, p.H,   \
-                  p.C, p.S, p.cb, p.units, p.packed, go, ro);                                            \
+                  p.C, p.S, p.cb, p.units, p.packed, go, ro);                                  \
     } while (0)
     // gate|up: 12 wavefronts (3 per SIMD; 4 weight blocks in flight fit
     // their registers); one tile: 16 (4 per SIMD, 7 of 112 blocks each, 4

@@ -30,6 +30,33 @@ extern std::atomic<bool> g_kernel_timing_on;
     } while (0)
 
 namespace si {
+// Something set up once on each GPU (a device past the 64th: on each call),
+// from any host thread: two that come first together both do it, which must
+// do no harm.  set(): whether it succeeded.
+class PerDevice {
+    std::atomic<uint64_t> done_{0};
+
+public:
+    template <class Set>
+    void once(int dev, Set set) {
+        const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
+        if (done_.load(std::memory_order_acquire) & bit) return;
+        if (set()) done_.fetch_or(bit, std::memory_order_release);
+    }
+};
+
+// Allows a kernel bytes of dynamic LDS, past the 64 KB it may have otherwise
+// (an attribute of the kernel on one GPU), before its launch on the current
+// one; a failure surfaces as the launch's error.
+inline void allow_lds(PerDevice &set, const void *kernel, int bytes) {
+    int dev = -1;
+    (void)hipGetDevice(&dev);
+    set.once(dev, [&] {
+        return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) ==
+               hipSuccess;
+    });
+}
+
 void launch_quantize_q8_aos(const float *src, void *dst, int count, hipStream_t st);
 void launch_quantize_q8_rows(const float *src, int rows, int k, int8_t *qs, uint16_t *d,
                              int16_t *s, hipStream_t st);
