@@ -360,13 +360,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p, uint32
 typedef __attribute__((address_space(3))) void lds_void;
 
 // One wavefront copy global -> LDS: lane l's 16 bytes at voff of r land at
-// lds + 16 l; a 2-byte copy lands zero-extended in the dword at lds + 4 l
-// (measured on MI355X); lds wavefront-uniform.
+// lds + 16 l; lds wavefront-uniform.
 __device__ __forceinline__ void lds_copy16(__amdgpu_buffer_rsrc_t r, uint8_t *lds, uint32_t voff) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 16, voff, 0, 0, 0);
-}
-__device__ __forceinline__ void lds_copy2(__amdgpu_buffer_rsrc_t r, uint8_t *lds, uint32_t voff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 2, voff, 0, 0, 0);
 }
 
 // Signed 8-bit 4-way dot product with int32 accumulate (v_dot4_i32_i8).
