@@ -489,7 +489,7 @@ int si_rope_kv_append(const si_shape_t *s, const float *qkv, int ldqkv, int ntok
     return check_launch("si_rope_kv_append");
 }
 
-// context splits, or what a causal prefill is sized by
+// context splits, or what a causal prefill is accepted by (it uses none)
 size_t si_attention_workspace(const si_shape_t *s, int nq, int max_ctx) {
     if (!s || nq <= 0 || max_ctx <= 0) return 0;
     const size_t a = attn_workspace_bytes(s->qheads, s->hdim, s->kvheads, nq, max_ctx);

@@ -434,9 +434,10 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
 // partner lane ^ 32), then
 //     O^T[d][row] += V^T[d][pos] . P^T[pos][row]     (v_mfma_f32_32x32x16_f16)
 // The running max and sum of a row then live in the lanes that hold its O^T
-// column, so the rescale is a per-lane multiply, and rare (below).  P is split into fp16 hi + lo halves like Q (an fp16-only P moves
-// outputs by ~1e-3 relative, enough to break the prefill == sequential decode
-// agreement the reference tests).
+// column, so the rescale is a per-lane multiply, and rare (below).  P is split
+// into fp16 hi + lo halves like Q (an fp16-only P moves outputs by ~1e-3
+// relative, enough to break the prefill == sequential decode agreement the
+// reference tests).
 //
 // Bound: the matrix pipe, 2 * (D/16 + D/16) instructions of ~33 cycles per
 // tile (1056 at D = 128) against ~115 VALU operations, 16 of them
@@ -445,10 +446,10 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
 // merge another 8 us.  (Issuing the next tile's scores, or the previous
 // tile's weighing, among the exponentials within a wavefront changed nothing:
 // 92 and 88 us against 87 at 7B x 2048; the second wavefront already fills
-// those gaps.  What helped was fewer VALU operations: 87 -> 77 us.)  K and V tiles are
-// copied global -> LDS by buffer loads that write LDS (no staging registers,
-// no transposition: V^T operands come from the transposing LDS read), their
-// 16-byte chunks permuted within each row on the way so that neither the
+// those gaps.  What helped was fewer VALU operations: 87 -> 77 us.)  K and V
+// tiles are copied global -> LDS by buffer loads that write LDS (no staging
+// registers, no transposition: V^T operands come from the transposing LDS read),
+// their 16-byte chunks permuted within each row on the way so that neither the
 // score operands (32 rows, one chunk) nor the transposing reads (4 rows, 4
 // chunks) meet in a bank.
 //
@@ -834,8 +835,9 @@ bool attn_prefill_supported(int qheads, int kvheads, int hdim, const uint16_t *k
 }
 
 // What si_attention_workspace states for a causal prefill: callers size (and
-// si_attention_static accepts or refuses) by it.  The kernel itself merges
-// in LDS and uses none.
+// si_attention and si_attention_static accept or refuse) by it, as when the
+// split tiles' states went through memory.  The kernel itself merges in LDS and
+// uses none.
 size_t attn_prefill_workspace_bytes(int qheads, int hdim, int ntok) {
     return (size_t)ntok * qheads * 2 * (hdim + 2) * sizeof(float);
 }

@@ -318,7 +318,8 @@ __device__ __forceinline__ void quant_block_pair16(const float (&x)[16], uint32_
 // the product with the reciprocal, corrected by its remainder.  Over all 2^32
 // gates (u = 1) the same bits as expf and the IEEE division but for 15 values,
 // at most 2 ulp apart, without their range checks: 21 instructions against
-// about 30.
+// about 30 (two of them choose the scale; the gate|up GEMMs' times are the same
+// without: 552 us at 2048 rows of 7B, 34.0 at 777 of 0.5B).
 __device__ __forceinline__ float swiglu(float g, float u) {
     const float gc = __builtin_amdgcn_fmed3f(g, -104.0f, 104.0f);  // e^-g is inf or 0 there
     const float t = __fmul_rn(gc, -1.44269502f), n = rintf(t);
