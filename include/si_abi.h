@@ -259,8 +259,7 @@ int si_rope_table(int npos, int hdim, float base, float *cos_host, float *sin_ho
  * Q8_0 quantization (planar, optional: pass NULL qs to skip).
  * workspace: si_attention_workspace bytes (fewer are taken where the batched
  * kernel states more chunks than the per-group one, which then runs; a causal
- * prefill is refused with fewer, though it leaves them untouched where kc and
- * vc are 16-byte aligned). */
+ * prefill is refused with fewer, though it leaves them untouched). */
 int si_attention(const si_shape_t *s, const float *q, int nq, const uint16_t *kc,
                  const uint16_t *vc, size_t kv_seq_stride, const int *ctx_dev,
                  int ctx0, int ctx_step, int max_ctx, float *attn, int8_t *qs,

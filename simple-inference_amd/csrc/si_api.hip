@@ -532,7 +532,7 @@ static int attention_impl(const char *what, const si_shape_t *s, const float *q,
     SI_REQUIRE(!qs || d, "%s: qs without d", what);
     SI_REQUIRE(ws_bytes >= attention_least(s, nq, max_ctx), "%s: workspace too small", what);
     if (!ctx_dev && ctx_step == 1 && kv_seq_stride == 0 && nq > 1 &&
-        attn_prefill_supported(s->qheads, s->kvheads, s->hdim, kc, vc))
+        attn_prefill_supported(s->qheads, s->kvheads, s->hdim))
         // causal prefill of one sequence: the flash kernel (query i at
         // cache row ctx0 - 1 + i)
         launch_attn_prefill(q, nq, s->qheads, s->kvheads, s->hdim, ctx0 - 1, kc, vc, attn, qs, d,
@@ -1418,7 +1418,7 @@ static int run_rows(si_layer *L, const float *x, int rows, uint16_t *kc, uint16_
                            kv_seq_stride, st);
         // :268-272: attention over the fp16 cache -> Q8
         mark(L, SI_PHASE_ATTENTION_Q8, st);
-        if (ctx_dev == nullptr && attn_prefill_supported(s.qheads, s.kvheads, s.hdim, kc, vc))
+        if (ctx_dev == nullptr && attn_prefill_supported(s.qheads, s.kvheads, s.hdim))
             launch_attn_prefill(L->q, rows, s.qheads, s.kvheads, s.hdim, pos0, kc, vc, L->attn,
                                 L->attq.qs, L->attq.d, L->attq.s, st);
         else

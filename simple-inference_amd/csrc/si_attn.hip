@@ -461,6 +461,8 @@ __global__ void __launch_bounds__(256) k_attn_decode_mfma(
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef _Float16 pf_h2 __attribute__((ext_vector_type(2)));
 typedef float pf_f2 __attribute__((ext_vector_type(2)));
+typedef uint32_t pf_u4 __attribute__((ext_vector_type(4)));
+typedef pf_u4 pf_u4u __attribute__((aligned(2)));  // at any fp16 address
 
 constexpr int PF_T = 32;      // query rows per wavefront, positions per K/V tile
 constexpr int PF_OPAD = 4;    // floats of padding per merged output row
@@ -522,7 +524,10 @@ __device__ __forceinline__ void pf_barrier() {
     asm volatile("" ::: "memory");
 }
 
-template <int D, int RT, int KW>
+// ASYNC: kc and vc are 16-byte aligned (and so is every row, a multiple of 64
+// bytes).  Otherwise the tiles come through registers, by loads that take any
+// address, and are in LDS when copy() returns.
+template <int D, int RT, int KW, bool ASYNC>
 __global__ void __launch_bounds__(RT * KW * 64) __attribute__((amdgpu_waves_per_eu(2)))
 k_attn_prefill(const float *__restrict__ q, int ntok, int qheads, int kvheads, int pos0,
                const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc, float scale2,
@@ -579,13 +584,29 @@ k_attn_prefill(const float *__restrict__ q, int ntok, int qheads, int kvheads, i
     }
     const auto copy = [&](const uint16_t *base, uint8_t *dst, int step, const int (&col)[TIW]) {
         const int kv0 = min(step * KW + kw, last / PF_T) * PF_T;  // past the range: the last tile
-        const __amdgpu_buffer_rsrc_t rs = buf_rsrc(base + (size_t)kv0 * kvd + g * D, 0x7fffffffu);
+        const uint16_t *src = base + (size_t)kv0 * kvd + g * D;
+        // rows past the last one read it again (masked out)
+        const auto at = [&](int i) {
+            return (uint32_t)(min(crow[i], last - kv0) * (kvd * 2) + col[i]);
+        };
+        uint8_t *const to = dst + kw * TB + 1024 * rt;
+        if constexpr (ASYNC) {
+            const __amdgpu_buffer_rsrc_t rs = buf_rsrc(src, 0x7fffffffu);
 #pragma unroll
-        for (int i = 0; i < TIW; ++i)
-            if (TI % RT == 0 || rt + RT * i < TI)
-                // rows past the last one read it again (masked out)
-                lds_copy16(rs, dst + kw * TB + 1024 * (rt + RT * i),
-                           (uint32_t)(min(crow[i], last - kv0) * (kvd * 2) + col[i]));
+            for (int i = 0; i < TIW; ++i)
+                if (TI % RT == 0 || rt + RT * i < TI) lds_copy16(rs, to + 1024 * RT * i, at(i));
+        } else {
+            pf_u4 x[TIW];
+#pragma unroll
+            for (int i = 0; i < TIW; ++i)
+                if (TI % RT == 0 || rt + RT * i < TI)
+                    x[i] = *(const pf_u4u *)((const uint8_t *)src + at(i));
+#pragma unroll
+            for (int i = 0; i < TIW; ++i)
+                if (TI % RT == 0 || rt + RT * i < TI)
+                    *(pf_u4 *)(to + 1024 * RT * i + 16 * lane) = x[i];
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
     };
     copy(kc, sb0, 0, ck);
     copy(vc, DB ? sb0 + KW * TB : sb1, 0, cv);
@@ -825,12 +846,8 @@ k_attn_prefill(const float *__restrict__ q, int ntok, int qheads, int kvheads, i
 
 // Causal prefill of ntok tokens at positions pos0.. of one sequence whose
 // cache rows 0..pos0+ntok-1 are in place (RoPE'd K, V).
-// The tiles are copied 16 bytes a lane straight into LDS, which takes aligned
-// rows (a row is a multiple of 64 bytes): a cache at any other address goes to
-// launch_attention's kernels, whose plain loads take it.
-bool attn_prefill_supported(int qheads, int kvheads, int hdim, const uint16_t *kc,
-                            const uint16_t *vc) {
-    return (((uintptr_t)kc | (uintptr_t)vc) & 15) == 0 && kvheads > 0 && qheads % kvheads == 0 && qheads / kvheads <= 16 &&
+bool attn_prefill_supported(int qheads, int kvheads, int hdim) {
+    return kvheads > 0 && qheads % kvheads == 0 && qheads / kvheads <= 16 &&
            (hdim == 32 || hdim == 64 || hdim == 96 || hdim == 128);
 }
 
@@ -863,25 +880,32 @@ void launch_attn_prefill(const float *q, int ntok, int qheads, int kvheads, int 
     //   12 heads of 128, 5000 (1876)         186    173    157         315
     const long rows = (long)ntok * per;
     const long tiles = (rows + 31) / 32 * kvheads;
-    const int rt = tiles < (hdim <= 64 ? 1024 : 512) ? 1 : hdim <= 64 || tiles < 1280 ? 2 : 4;
+    // Caches off a 16-byte boundary, which the copies into LDS do not take:
+    // two tiles by two ways throughout, through registers (us a call, aligned |
+    // this | the per-query kernels: 0.5B 512 tokens 8.0 | 12.4 | 19.1, 7B 333
+    // after 1500 31.9 | 47.9 | 118, 7B 2048 75.8 | 83.5 | 339).
+    const bool async = (((uintptr_t)kc | (uintptr_t)vc) & 15) == 0;
+    const int rt = !async                              ? 2
+                   : tiles < (hdim <= 64 ? 1024 : 512) ? 1
+                   : hdim <= 64 || tiles < 1280        ? 2
+                                                       : 4;
     const dim3 grid((unsigned)((rows + 32 * rt - 1) / (32 * rt) * kvheads));
-#define PF_CALL(DIM, RT, KW)                                                                 \
-    SI_LAUNCH((k_attn_prefill<DIM, RT, KW>), grid, dim3(RT * KW * 64), 0, st, q, ntok, qheads, \
-              kvheads, pos0, kc, vc, scale2, attn, qs, qd, bsum)
-#define PF_DIM(DIM)                        \
-    switch (rt) {                          \
-        case 1: PF_CALL(DIM, 1, 4); break; \
-        default: PF_CALL(DIM, 2, 2);       \
-    }
+#define PF_CALL(DIM, RT, KW, ASYNC)                                                         \
+    SI_LAUNCH((k_attn_prefill<DIM, RT, KW, ASYNC>), grid, dim3(RT * KW * 64), 0, st, q, ntok, \
+              qheads, kvheads, pos0, kc, vc, scale2, attn, qs, qd, bsum)
+#define PF_DIM(DIM)                                \
+    if (!async) PF_CALL(DIM, 2, 2, false);         \
+    else if (rt == 1) PF_CALL(DIM, 1, 4, true);    \
+    else PF_CALL(DIM, 2, 2, true)
     switch (hdim) {
         case 32: PF_DIM(32); break;
         case 64: PF_DIM(64); break;
         case 96:
-            if (rt == 4) PF_CALL(96, 4, 2);
+            if (rt == 4) PF_CALL(96, 4, 2, true);
             else PF_DIM(96);
             break;
         default:
-            if (rt == 4) PF_CALL(128, 4, 2);
+            if (rt == 4) PF_CALL(128, 4, 2, true);
             else PF_DIM(128);
             break;
     }

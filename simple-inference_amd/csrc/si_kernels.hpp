@@ -249,9 +249,7 @@ void launch_attention(const float *q, int nq, int qheads, int kvheads, int hdim,
                       const int *ctx_dev, int ctx0, int ctx_step, int max_ctx, float *attn,
                       int8_t *qs, uint16_t *d, int16_t *bsum, void *workspace, size_t ws_bytes,
                       hipStream_t st, KvPages pg = KvPages(), int kv_row = 0);
-// Whether launch_attn_prefill takes the shape and these cache pointers.
-bool attn_prefill_supported(int qheads, int kvheads, int hdim, const uint16_t *kc,
-                            const uint16_t *vc);
+bool attn_prefill_supported(int qheads, int kvheads, int hdim);
 size_t attn_prefill_workspace_bytes(int qheads, int hdim, int ntok);
 void launch_attn_prefill(const float *q, int ntok, int qheads, int kvheads, int hdim, int pos0,
                          const uint16_t *kc, const uint16_t *vc, float *attn, int8_t *qs,

@@ -62,30 +62,36 @@ def test_prefill_attention_edges(qh, kv, d, n, prefix):
 
 
 @pytest.mark.parametrize("offset", [0, 1, 4, 8])
-@pytest.mark.parametrize("qh,kv,d,n,prefix", [(14, 2, 64, 5, 30), (12, 2, 128, 33, 7)])
+@pytest.mark.parametrize("qh,kv,d,n,prefix", [(14, 2, 64, 5, 30), (12, 2, 128, 33, 7),
+                                              (3, 1, 96, 43, 64), (5, 5, 32, 32, 32),
+                                              (64, 32, 96, 300, 3), (32, 32, 128, 1300, 0)])
 def test_prefill_attention_cache_address(qh, kv, d, n, prefix, offset):
-    """A cache that starts off a 16-byte boundary: the copies into LDS do not take
-    it, the kernels with plain loads do; the same values within the bound above
-    of both."""
+    """A cache that starts off a 16-byte boundary, which the copies into LDS do not
+    take: the same kernel with its tiles through registers, and the same values
+    within the bound above of both."""
     import torch
     g = torch.Generator(device="cuda").manual_seed(qh + n)
     q = torch.randn(n, qh, d, generator=g, device="cuda")
     rows = (prefix + n) * kv * d
     k, v = (torch.randn(rows, generator=g, device="cuda").half() for _ in range(2))
-    kb, vb = (torch.zeros(rows + 16, dtype=torch.float16, device="cuda") for _ in range(2))
+    # (no row past the last is weighed: what lies there would be seen)
+    kb, vb = (torch.full((rows + 16,), float("nan"), dtype=torch.float16, device="cuda")
+              for _ in range(2))
     kb[offset:offset + rows], vb[offset:offset + rows] = k, v
     s = si_amd.make_shape(32, qh, kv, d)
     need = si_amd.lib().si_attention_workspace(ctypes.byref(s), n, prefix + n)
     ws = empty((need,), torch.uint8)
     outs, names = [], []
-    for kc, vc in ((k, v), (kb[offset:], vb[offset:])):
+    for kc, vc in ((k, v), (kb[offset:], v), (k, vb[offset:]), (kb[offset:], vb[offset:])):
         out = empty((n, qh, d), torch.float32)
         names.append(si_amd.kernel_times_ms("k_", lambda: si_amd.call(
             "si_attention", ctypes.byref(s), si_amd.ptr(q), n, si_amd.ptr(kc), si_amd.ptr(vc), 0,
             None, prefix + 1, 1, prefix + n, si_amd.ptr(out), None, None, None, si_amd.ptr(ws),
             need, si_amd.stream_handle()))[0][0])
         outs.append(out.double())
-    assert names[0].startswith("k_attn_prefill")
-    assert names[1].startswith("k_attn_prefill") == (offset % 8 == 0), names[1]
-    err = (outs[0] - outs[1]).abs().amax(2) / outs[0].abs().amax(2)
-    assert err.max().item() < 2e-5
+    by_registers = "k_attn_prefill<%d, 2, 2, false>" % d
+    assert names[0].startswith("k_attn_prefill") and names[0] != by_registers
+    for name, out in zip(names[1:], outs[1:]):
+        assert name == (names[0] if offset % 8 == 0 else by_registers), names
+        err = (outs[0] - out).abs().amax(2) / outs[0].abs().amax(2)
+        assert err.max().item() < 2e-5
