@@ -868,7 +868,17 @@ struct RowsLds {
 };
 
 // RAW (si_attention): qkv holds rotated queries only ([nq][qheads * D]) and
-// every position's row is in the cache: no rotation, nothing appended.
+// every position's row is in the cache: no rotation, nothing appended.  The
+// chunks are the longest context's share of the grid, no more than the given
+// chunk (max_ctx's): max_ctx may be a server's limit far above the contexts,
+// each of which one workgroup would then walk alone.  us a call, per-group
+// kernel | max_ctx's chunks | this: 7B heads, 64 queries, contexts of 300 under
+// 4096 27.5 | 40.6 | 18.9, of 4000 under 32768 279 | 401 | 103, of 64 under 4096
+// 14.1 | 16.2 | 14.0; 0.5B heads, 32 of 100-2000 under 32768 60.7 | 45.3 | 10.4;
+// with a context as long as max_ctx 45-70 us calls take up to 0.6 more for the
+// maximum.  (A share of each query's own context instead: 7B, 48 of 200-4096,
+// cold, 57.6 -> 59.1: its short ones, cut finer, leave the long ones alone at
+// the end.)
 template <int D, int G, bool FINAL, bool PAGED, bool RAW>
 __global__ void __launch_bounds__(256) k_dec_attn_rows(
     const float *__restrict__ qkv, int ldqkv, int qheads, const float *__restrict__ rc,
@@ -904,6 +914,17 @@ __global__ void __launch_bounds__(256) k_dec_attn_rows(
     int ctx = ctx_dev ? ctx_dev[qi] : ctx0 + qi * ctx_step;
     ctx = min(ctx, max_ctx);
     const int pnew = ctx - 1;  // < 0: empty context (device-supplied only)
+    if (RAW && ns > 1) {  // (gridDim.y < 512 then)
+        const int nq = gridDim.y;
+        int most = ctx0 + (nq - 1) * ctx_step;
+        if (ctx_dev) {
+            most = 0;
+            for (int i = lane; i < nq; i += 64) most = max(most, ctx_dev[i]);
+            most = __builtin_amdgcn_readfirstlane(wave_max_i(most));
+        }
+        const int share = (min(most, max_ctx) + ns - 1) / ns;
+        chunk = min(chunk, max(2 * ROWS, (share + DA_TILE - 1) / DA_TILE * DA_TILE));
+    }
     const int p0 = sp * chunk;
     const int p1 = min(ctx, p0 + chunk);
     // rows the loads may touch: known at launch, so the first loads need not

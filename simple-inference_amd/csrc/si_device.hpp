@@ -170,6 +170,14 @@ __device__ __forceinline__ float wave_max(float v) {
     v = fmaxf(v, swap16_f(v));
     return fmaxf(v, swap32_f(v));
 }
+__device__ __forceinline__ int wave_max_i(int v) {
+    v = max(v, dpp_i<DPP_XOR1>(v));
+    v = max(v, dpp_i<DPP_XOR2>(v));
+    v = max(v, dpp_i<DPP_ROR4>(v));
+    v = max(v, dpp_i<DPP_ROR8>(v));
+    v = max(v, swap16_i(v));
+    return max(v, swap32_i(v));
+}
 __device__ __forceinline__ double dpp_d_add(double v, int which) {
     const long long b = __double_as_longlong(v);
     int lo = (int)b, hi = (int)(b >> 32);

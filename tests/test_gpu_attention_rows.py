@@ -120,3 +120,47 @@ def test_attention_rows_host_contexts():
                 k.stride(0), None, ctx0, step, ctx[-1], si_amd.ptr(out), None, None, None,
                 si_amd.ptr(ws), need, si_amd.stream_handle())
     _check(out, _want(q, k, v, ctx, qh // kv), ctx)
+
+
+@pytest.mark.parametrize("qh,kv,d,cap,ctx", [
+    (28, 4, 128, 4096, [300, 1, 0, 32, 33, 299, 16, 17, 64, 65, 128, 200]),
+    (28, 4, 128, 700, [100 + i for i in range(80)]),  # more queries than lanes, the longest last
+    (14, 2, 64, 9000, [1000, 64, 65, 1, 0, 999, 500, 130]),
+    (5, 1, 32, 20000, [0] * 8 + [5]),
+    (16, 1, 96, 6000, [700, 1, 255, 256, 257, 128, 129, 2]),
+    (12, 2, 128, 4096, [0] * 9),
+])
+@pytest.mark.parametrize("on_host", [False, True])
+def test_attention_rows_short_contexts(qh, kv, d, cap, ctx, on_host):
+    """Contexts far below max_ctx: the longest one's chunks are its share of the
+    grid (max_ctx's share would leave it to one workgroup), seen in the partial
+    states (outputs, then maxima: -inf for an empty chunk)."""
+    import torch
+    n = len(ctx)
+    if on_host:
+        ctx = [10 + 3 * i for i in range(n)]
+    g = torch.Generator(device="cuda").manual_seed(cap)
+    q = torch.randn(n, qh, d, generator=g, device="cuda")
+    k, v = (torch.full((n, cap, kv, d), float("nan"), dtype=torch.float16, device="cuda")
+            for _ in range(2))
+    for i, c in enumerate(ctx):
+        for t in (k, v):
+            t[i, :c] = torch.randn(c, kv, d, generator=g, device="cuda").half()
+    s = si_amd.make_shape(32, qh, kv, d)
+    cd = None if on_host else torch.tensor(ctx, dtype=torch.int32, device="cuda")
+    need = si_amd.lib().si_attention_workspace(ctypes.byref(s), n, cap)
+    ws = torch.full((need // 4,), float("nan"), device="cuda")
+    out = empty((n, qh, d), torch.float32)
+    ran = si_amd.kernel_times_ms("k_", lambda: si_amd.call(
+        "si_attention", ctypes.byref(s), si_amd.ptr(q), n, si_amd.ptr(k), si_amd.ptr(v),
+        k.stride(0), si_amd.ptr(cd), 10, 3, cap, si_amd.ptr(out), None, None, None,
+        si_amd.ptr(ws), need, si_amd.stream_handle()))
+    assert ran[0][0].startswith("k_dec_attn_rows"), ran
+    _check(out, _want(q, k, v, ctx, qh // kv), ctx)
+    step = 16 * (4 // kv)
+    ns = min(-(-cap // (4 * step)), -(-512 // n), 31)
+    top = ws[n * qh * ns * d:][:n * qh * ns].view(n, qh, ns)
+    up16 = lambda c: (c + 15) // 16 * 16
+    chunk = min(up16(-(-cap // ns)), max(2 * step, up16(-(-max(ctx) // ns))))
+    for i, c in enumerate(ctx):
+        assert bool((torch.isfinite(top[i]).sum(1) == -(-c // chunk)).all()), (i, c, chunk)
